@@ -663,16 +663,14 @@ int pi05w4a4_gemm_e3m2(const void* q6, const float* sa, int64_t m, int32_t k, in
   if (q6 == nullptr || sa == nullptr) return fail(PI05W4A4_EINVAL, "null activation codes or scales");
   if (!aligned(q6, 16) || !aligned(sa, 4))
     return fail(PI05W4A4_EINVAL, "q6 must be 16-byte aligned, sa 4-byte aligned");
-  // Tiles: 112 x 256 (GELU: 112 x 128 gate + up) when they give at least 1.5 workgroups per
-  // CU, else 32 x 128 (the narrow GEMMs: QKV, o).
+  // Tiles: the main tile (16 mi x 256 outputs; GELU: 128 gate + up) when 112-row tiles give at
+  // least 1.5 workgroups per CU, else 32 x 128 (the narrow GEMMs: QKV, o).  The main tile's
+  // height is the smallest multiple of 16 rows that covers M in ceil(M / 112) equal tiles (at
+  // 200 rows 112, at 130 rows 80).
   const int64_t cus = w4a4::device_cu_count();
   const int64_t m7 = cdiv(m, 112);
-  int64_t n7 = 0, n2 = 0;
-  for (int g = 0; g < ngroups; ++g) {
-    n7 += cdiv(n[g], gelu_up != 0 ? 128 : 256);
-    n2 += cdiv(n[g], 128);
-  }
-  if (gelu_up != 0) n7 = cdiv(n[0], 128);
+  int64_t n7 = 0;
+  for (int g = 0; g < ngroups; ++g) n7 += cdiv(n[g], 256);
   const bool narrow = gelu_up == 0 && 2 * m7 * n7 < 3 * cus;
   const int tile_cfg = narrow ? w4a4::kCfg2x2 : w4a4::kCfg7x4;
   const int64_t mtiles = narrow ? cdiv(m, 32) : m7;
@@ -696,6 +694,8 @@ int pi05w4a4_gemm_e3m2(const void* q6, const float* sa, int64_t m, int32_t k, in
   }
   p.ntiles = gelu_up != 0 ? static_cast<int32_t>(cdiv(n[0], tile_cols)) : tile_begin;
   p.mtiles = static_cast<int32_t>(mtiles);
+  p.mi = static_cast<int32_t>(std::max<int64_t>(4, cdiv(m, 16 * m7)));
+  p.mgroup = static_cast<int32_t>(cdiv(mtiles, cdiv(mtiles, 16)));  // equal groups of at most 16 (2.8 MB at K = 2048)
   p.ksplit = 1;
   p.kblocks_per_split = w4a4::kblocks128(k);
   p.mblocks = static_cast<int32_t>(cdiv(m, 16));

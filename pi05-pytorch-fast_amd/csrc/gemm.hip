@@ -149,6 +149,14 @@ __device__ __forceinline__ _Float16 dequant(float acc, float sa, float sw) {
 // E3M2 operand of one fragment from six consecutive dwords (the upper two are unused).
 __device__ __forceinline__ v8i e3m2_op(v4i lo, int d4, int d5) { return v8i{lo.x, lo.y, lo.z, lo.w, d4, d5, 0, 0}; }
 
+}  // namespace
+}  // namespace w4a4
+
+#include "gemm_e3m2_tile.h"
+
+namespace w4a4 {
+namespace {
+
 // RoPE of four dimension pairs (d, d + 128), each product and sum rounded to fp16 as
 // torch's (x * cos) + (rotate_half(x) * sin) on fp16 tensors (attention.hip's rope_pair).
 __device__ __forceinline__ void rope4(half4& lo, half4& hi, half4 clo, half4 chi, half4 slo, half4 shi) {
@@ -270,25 +278,29 @@ __device__ __forceinline__ void down_quant_role(const GemmParams& p, char* lds) 
 
 // E3M2: both operands in the E3M2 layouts of w4a4_internal.h (q6 fragments, w6 column
 // pairs) and v_mfma_f32_16x16x128_f8f6f4: one MFMA per fragment pair and 128-deep k block
-// (half the int8 MFMA issue time for the same work) and no unpack.  Its operands take
-// 1.5x the bytes of INT4 codes, and a CU's vector-memory path delivers about one 64-lane
-// 16-byte load per ~28 clocks, so the A fragments, which the four waves of the workgroup
-// share, are staged once per workgroup in a double-buffered LDS tile by direct
-// global-to-LDS loads (11 1 KB chunks per k block, dealt over the waves), and only the B
-// column pairs stream per wave (three 16-byte loads per pair).  Step kb: wait for this
-// wave's loads, workgroup barrier (every wave's A(kb) chunks are in LDS; every wave has
-// read slot kb + 1 in step kb - 1), read A(kb) from LDS, issue A(kb + 1) and B(kb + 1),
-// then the 28 MFMAs.  All LDS reads of a step precede its LDS-bound loads, so the
-// compiler's conservative wait on those loads never lands before a read.  The fp32
-// accumulators start at zero and end at acc exactly (no 16x factor, no corrections).
+// (half the int8 MFMA issue time for the same work) and no unpack.  NI == 4 runs the main
+// tile of gemm_e3m2_tile.h; the code below is the narrow form (32 x 128 tiles), whose A
+// fragments are staged once per workgroup in a double-buffered LDS tile by direct
+// global-to-LDS loads and whose B column pairs stream per wave (three 16-byte loads per
+// pair).  Step kb: wait for this wave's loads, workgroup barrier (every wave's A(kb) chunks
+// are in LDS; every wave has read slot kb + 1 in step kb - 1), read A(kb) from LDS, issue
+// A(kb + 1) and B(kb + 1), then the MFMAs.  All LDS reads of a step precede its LDS-bound
+// loads, so the compiler's conservative wait on those loads never lands before a read.  The
+// fp32 accumulators start at zero and end at acc exactly (no 16x factor, no corrections).
 template <int MI, int NI, int NWAVES, int KW, bool GELU, int RING, int WPE, bool QKV_PREP = false, bool QFUSE = false,
           bool E3M2 = false, bool QPRO = false, int NKB = 0>
 __global__ __launch_bounds__(64 * NWAVES) __attribute__((amdgpu_waves_per_eu(WPE))) void gemm_w4a4_kernel(const GemmParams p) {
+  if constexpr (E3M2 && NI == 4) {
+    // The main E3M2 tile (gemm_e3m2_tile.h).
+    __shared__ __align__(16) char lds_tile[E3m2Tile<MI, GELU>::kLds];
+    e3m2_tile<MI, GELU>(p, lds_tile, kGeluFix.v);
+    return;
+  } else {
   static_assert(!(GELU && QKV_PREP), "the attention prep is a fp16 epilogue");
   static_assert(!QPRO || (MI == 1 && NWAVES == 4 && KW == 4 && RING >= 3 && !GELU && !QFUSE && !E3M2),
                 "the quant prologue runs in the four K-split waves of one 16-row block");
-  static_assert(!E3M2 || (NI % 2 == 0 && NWAVES == 4 && KW == 1 && !QFUSE && (!GELU || NI == 4)),
-                "E3M2 operands: four waves along N, whole column pairs per wave");
+  static_assert(!E3M2 || (NI % 2 == 0 && NWAVES == 4 && KW == 1 && !QFUSE && !GELU && !QKV_PREP),
+                "narrow E3M2 tiles: four waves along N, whole column pairs per wave, plain outputs");
   static_assert(!GELU || (NI % 2 == 0), "GELU pairing needs an even NI");
   static_assert(NWAVES % KW == 0 && (KW & (KW - 1)) == 0, "waves split as NW x KW");
   constexpr int NW = NWAVES / KW;
@@ -1137,6 +1149,7 @@ __global__ __launch_bounds__(64 * NWAVES) __attribute__((amdgpu_waves_per_eu(WPE
       }
     }
   }
+  }
 }
 
 // Sum the split-K partials and apply the epilogue.  Each thread owns 4 consecutive
@@ -1303,23 +1316,36 @@ hipError_t launch_gemm_gelu_quant(const GemmParams& p, int nquant, hipStream_t s
 }
 
 hipError_t launch_gemm_e3m2(const GemmParams& p, int tile_cfg, hipStream_t stream) {
-  if (p.ksplit != 1 || (p.mode != kEpiFp16 && p.mode != kEpiGeluUp)) return hipErrorInvalidValue;
+  if (p.ksplit != 1 || (p.mode != kEpiFp16 && p.mode != kEpiGeluUp) || p.rope_group > 0) return hipErrorInvalidValue;
   const bool gelu = p.mode == kEpiGeluUp;
-  const bool prep = p.rope_group > 0;
-  if ((gelu && (prep || p.res != nullptr || tile_cfg != kCfg7x4)) || (tile_cfg != kCfg7x4 && tile_cfg != kCfg2x2))
-    return hipErrorInvalidValue;
-  const dim3 grid(static_cast<unsigned>(p.ntiles) * static_cast<unsigned>(p.mtiles));
-  if (gelu)
-    gemm_w4a4_kernel<7, 4, 4, 1, true, 2, 2, false, false, true><<<grid, 256, 0, stream>>>(p);
-  else if (tile_cfg == kCfg7x4 && !prep)
-    gemm_w4a4_kernel<7, 4, 4, 1, false, 2, 2, false, false, true><<<grid, 256, 0, stream>>>(p);
-  else if (tile_cfg == kCfg7x4)
-    gemm_w4a4_kernel<7, 4, 4, 1, false, 2, 2, true, false, true><<<grid, 256, 0, stream>>>(p);
-  else if (!prep)
-    gemm_w4a4_kernel<2, 2, 4, 1, false, 2, 2, false, false, true><<<grid, 256, 0, stream>>>(p);
-  else
-    gemm_w4a4_kernel<2, 2, 4, 1, false, 2, 2, true, false, true><<<grid, 256, 0, stream>>>(p);
-  return hipGetLastError();
+  if (gelu && (p.res != nullptr || tile_cfg != kCfg7x4)) return hipErrorInvalidValue;
+  const unsigned tiles = static_cast<unsigned>(p.ntiles) * static_cast<unsigned>(p.mtiles);
+  if (tile_cfg == kCfg2x2) {
+    gemm_w4a4_kernel<2, 2, 4, 1, false, 2, 2, false, false, true><<<dim3(tiles), 256, 0, stream>>>(p);
+    return hipGetLastError();
+  }
+  if (tile_cfg != kCfg7x4) return hipErrorInvalidValue;
+  // The main tile: two workgroups per CU walk the tiles.  The walk goes on with the next
+  // tile's k blocks in the same ring positions, so it needs an even count of them (and four,
+  // the loads' lead); otherwise every workgroup gets one tile.
+  const int nkb = kblocks128(p.k);
+  const unsigned slots = 2u * static_cast<unsigned>(device_cu_count());
+  const dim3 grid((nkb % 2 == 0 && nkb >= 4 && tiles > slots) ? slots : tiles);
+  auto launch = [&](auto mi) {
+    constexpr int MI = decltype(mi)::value;
+    if (gelu)
+      gemm_w4a4_kernel<MI, 4, 4, 1, true, 2, 2, false, false, true><<<grid, 256, 0, stream>>>(p);
+    else
+      gemm_w4a4_kernel<MI, 4, 4, 1, false, 2, 2, false, false, true><<<grid, 256, 0, stream>>>(p);
+    return hipGetLastError();
+  };
+  switch (p.mi) {
+    case 4: return launch(std::integral_constant<int, 4>{});
+    case 5: return launch(std::integral_constant<int, 5>{});
+    case 6: return launch(std::integral_constant<int, 6>{});
+    case 7: return launch(std::integral_constant<int, 7>{});
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t launch_gelu_up(const void* g, const void* u, int64_t n, void* y, hipStream_t stream) {

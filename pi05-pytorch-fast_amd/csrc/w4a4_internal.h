@@ -45,6 +45,8 @@ struct GemmParams {
   GemmGroup g[kMaxGroups];
   int32_t ntiles;     // total n-tiles over the groups
   int32_t mtiles;
+  int32_t mi;         // E3M2 main tile: row fragments per wave (the tile has 16 mi rows)
+  int32_t mgroup;     // E3M2 main tile: m-tiles per group of the tile order
   int32_t ksplit;     // number of K slices
   int32_t kblocks_per_split;  // 128-deep k blocks per K slice
   int32_t mode;
@@ -240,10 +242,9 @@ hipError_t launch_repack_e3m2(const int32_t* w_mfma, int32_t n, int32_t k, int32
 hipError_t launch_quantize_e3m2(const void* x, const void* nw, float eps, int unit_offset, int64_t m,
                                 int32_t k, void* q6, float* sa, float inv_sqrt_k, hipStream_t stream,
                                 const CacheWarmParams* warm = nullptr);
-// GEMM on E3M2 operands, tile_cfg kCfg7x4 (112 x 256 workgroup tiles, GELU pairs or
-// plain) or kCfg2x2 (32 x 128), four waves along N, no K split; modes kEpiFp16 (1..3
-// groups, optional residual or QKV attention prep) and kEpiGeluUp; p.q points at q6, the
-// groups' w at w6.
+// GEMM on E3M2 operands, tile_cfg kCfg7x4 (the main tile, 16 p.mi x 256 outputs, GELU pairs or
+// plain, optional residual) or kCfg2x2 (32 x 128, plain), four waves along N, no K split;
+// modes kEpiFp16 (1..3 groups) and kEpiGeluUp; p.q points at q6, the groups' w at w6.
 hipError_t launch_gemm_e3m2(const GemmParams& p, int tile_cfg, hipStream_t stream);
 // 16 x 32 tiles whose four waves split K (K = 2048, 1 <= M <= kQproMaxRows, one K slice,
 // fp16 epilogue without the attention prep), the activation quant of p.xpro in every

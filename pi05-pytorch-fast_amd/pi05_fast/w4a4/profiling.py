@@ -244,10 +244,10 @@ def _gemm_e3m2_bytes(m: int, k: int, n: int, out_bytes: float) -> float:
 # E3M2, QPRO, NKB>, fwht_quant_kernel<LOGK, LOGT, ROWS, NORM, E3M2>.
 _M = 776
 TRAFFIC_CLASSES = {
-    "gate_up_gelu": ("gemm_w4a4_kernel<7, 4, 4, 1, true, 2, 2, false, false, true, false, 0>", 896,
+    "gate_up_gelu": ("gemm_w4a4_kernel<7, 4, 4, 1, true, 2, 2, false, false, true, false, 0>", 512,
                      _gemm_e3m2_bytes(_M, 2048, 32768, 2.0 * _M * 16384),
                      "E3M2 codes A 1.19 MB + gate and up weights 50.33 MB + scales; fp16 h 25.43 MB"),
-    "gate_up": ("gemm_w4a4_kernel<7, 4, 4, 1, false, 2, 2, false, false, true, false, 0>", 896,
+    "gate_up": ("gemm_w4a4_kernel<7, 4, 4, 1, false, 2, 2, false, false, true, false, 0>", 512,
                 _gemm_e3m2_bytes(_M, 2048, 32768, 2.0 * _M * 32768),
                 "E3M2 codes A 1.19 MB + weights 50.33 MB + scales; fp16 gate and up 50.86 MB"),
     "gate_up_gelu_int4": ("gemm_w4a4_kernel<7, 4, 4, 1, true, 2, 2, false, false, false, false, 0>", 896,
