@@ -188,8 +188,8 @@ __device__ __forceinline__ int64_t vfrag_slot(int d, int t0, int nst) {
 // completion after its stores (release at agent scope: the workgroups of one row block run
 // on all eight XCDs), and a quant workgroup takes rows in increasing order from a shared
 // counter, waits (bounded) for the row's m-tile, acquires, and runs the row through the
-// K = 16384 quantizer of the standalone kernel (fwht_quant_row, 256 threads, one 68 KB LDS
-// row), so the codes are those of pi05w4a4_quantize bit for bit.  The tiles are dealt
+// K = 16384 quantizer of the standalone kernel (fwht_quant_row16k, 256 threads, 68 KB of
+// LDS), so the codes are those of pi05w4a4_quantize bit for bit.  The tiles are dealt
 // m-tile-major within each XCD, so the first round of tiles completes whole row blocks and
 // the quant workgroups that fill the slots left idle by the partial last round of tiles
 // have rows to work on while it runs.
@@ -199,15 +199,12 @@ __device__ __forceinline__ int64_t vfrag_slot(int d, int t0, int nst) {
 // target.  The wait is bounded anyway (spin_limit rounds of s_sleep): one that runs out
 // leaves the row unquantized, sets *qstatus for the host and the workgroup leaves.
 constexpr int kQuantLogK = 14;
-constexpr int kQuantLogT = 8;
-constexpr int kQuantR = 1 << (kQuantLogK - kQuantLogT);                             // 64 values per thread
-constexpr int kQuantLrow = (1 << kQuantLogK) + 4 * ((1 << kQuantLogK) / kQuantR);   // LDS floats per row
-constexpr int kQuantLdsBytes = kQuantLrow * 4 + 64;                                 // + reductions, broadcast
+constexpr int kQuantLdsBytes = kRow16kLds<false> * 4 + 64;  // the row's LDS, reductions, broadcast
 
 template <int TILE_ROWS>
 __device__ __forceinline__ void down_quant_role(const GemmParams& p, char* lds) {
   float* const L = reinterpret_cast<float*>(lds);
-  float* const red = L + kQuantLrow;
+  float* const red = L + kRow16kLds<false>;
   int* const ired = reinterpret_cast<int*>(red + 4);
   int* const bcast = ired + 4;
   const int t = threadIdx.x;
@@ -252,15 +249,11 @@ __device__ __forceinline__ void down_quant_role(const GemmParams& p, char* lds) 
     }
     // The row block's stores happen-before the counts this thread saw: acquire them.
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    float v[kQuantR];
-    const _Float16* xr = h + static_cast<int64_t>(row) * (1 << kQuantLogK) + t * kQuantR;
+    row16k_in xv[8];
+    const _Float16* xr = h + static_cast<int64_t>(row) * (1 << kQuantLogK) + t * 64;
 #pragma unroll
-    for (int c = 0; c < kQuantR / 8; ++c) {
-      const half8 hv = *reinterpret_cast<const half8*>(xr + 8 * c);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[8 * c + e] = static_cast<float>(hv[e]);
-    }
-    fwht_quant_row<kQuantLogK, kQuantLogT>(v, L, red, ired, t, row, p.dq, p.dsa, qcorr, p.dinv_sqrt_k);
+    for (int c = 0; c < 8; ++c) xv[c] = *reinterpret_cast<const row16k_in*>(xr + 8 * c);
+    fwht_quant_row16k<false>(xv, L, red, ired, t, row, p.dq, p.dsa, qcorr, p.dinv_sqrt_k);
     __syncthreads();  // the next row reuses L, red and bcast
   }
   // The last quant workgroup to leave returns the control block to zero for the next launch

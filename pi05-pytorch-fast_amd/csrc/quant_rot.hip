@@ -29,6 +29,20 @@
 namespace w4a4 {
 namespace {
 
+// Workgroup b's group of ROWS rows.  A 128-byte line of the code fragments holds pieces of 8
+// rows, and workgroup b runs on XCD b % 8: taken in order, the rows of a 16-row block would be
+// written from all eight L2s, each line in eight partial writes.  So XCD x takes the 16-row
+// blocks x, x + 8, ... (of whole runs of 8 blocks; the last M % 128 rows keep their order).
+// Measured (in order / so): K = 16384 half rows at 6208 rows 112 / 70 us, whole rows at 512 rows
+// 11.7 / 9.1 us; K = 2048 at 6208 rows 13.6 / 13.2 us.
+template <int ROWS>
+__device__ __forceinline__ uint32_t xcd_row_group(uint32_t b, uint32_t m) {
+  constexpr uint32_t kPer = 16 / ROWS;  // workgroups per 16-row block
+  if (b >= (m >> 7) * (8 * kPer)) return b;
+  const uint32_t i = b >> 3;
+  return ((i / kPer) * 8 + (b & 7)) * kPer + i % kPer;
+}
+
 template <int T>
 __device__ __forceinline__ float block_max(float v, float* red) {
   v = wave_max(v);
@@ -160,10 +174,9 @@ __global__ __launch_bounds__(T) void quant_rot_kernel(const _Float16* __restrict
   if (t == 0) qcorr[row] = -8 * s16;
 }
 
-// Register-FFT form of the same transform for K = 2^LOGK, T = 2^LOGT threads per row
-// (fwht_quant_row in quant_row.h): each thread loads R = K/T consecutive values (one
-// coalesced 2R-byte load) and the passes run in registers with LDS transposes between
-// them.  ROWS rows per workgroup; with T = 64 every row belongs to one wave and the
+// Register-FFT form of the same transform for K = 2^LOGK, T = 2^LOGT threads per row: each
+// thread loads R = K/T consecutive values (one coalesced 2R-byte load).
+// ROWS rows per workgroup; with T = 64 every row belongs to one wave and the
 // passes need no workgroup barrier.
 // NORM: the row is first replaced by its RMSNorm (transformers' GemmaRMSNorm,
 // modeling_gemma.py:64-78, with weight nw and the (1 + w) offset when unit_offset):
@@ -172,9 +185,9 @@ __global__ __launch_bounds__(T) void quant_rot_kernel(const _Float16* __restrict
 // with ss summed per lane over its R consecutive elements in order, then over the 64
 // lanes by the xor butterfly 32, 16, .., 1 (the oracle restates this order exactly), and
 // the fp16 h is what gets rotated and quantized, as if the norm's output had been stored.
-// E3M2 (K = 2048): the codes are written as E3M2 fragments (q points at the q6 buffer).
-template <int LOGK, int LOGT, int ROWS, bool NORM = false, bool E3M2 = false>
-__global__ __launch_bounds__(ROWS << LOGT) void fwht_quant_kernel(
+// E3M2: the codes are written as E3M2 fragments (q points at the q6 buffer).
+template <int LOGK, int LOGT, int ROWS, bool NORM = false, bool E3M2 = false, bool HALF = false>
+__global__ __launch_bounds__(ROWS << LOGT, HALF ? 3 : 1) void fwht_quant_kernel(
     const _Float16* __restrict__ x, int64_t m, int32_t* __restrict__ q, float* __restrict__ sa,
     int32_t* __restrict__ qcorr, float inv_sqrt_k, const _Float16* __restrict__ nw = nullptr,
     float eps = 0.0f, int unit_offset = 0, const CacheWarmParams warm = CacheWarmParams{}) {
@@ -190,24 +203,30 @@ __global__ __launch_bounds__(ROWS << LOGT) void fwht_quant_kernel(
       return;
     }
   }
-  constexpr int LROW = K + 4 * (K / R);  // LDS floats per row (4 pad floats per R)
+  static_assert(T == 64 || (LOGK == 14 && LOGT == 8), "one wave per row, or K = 16384 in 256 threads");
   // One wave per row (T == 64) runs in registers only (fwht_quant_row_wave).
-  __shared__ __align__(16) float lds[T == 64 ? 1 : ROWS * LROW];
+  __shared__ __align__(16) float lds[T == 64 ? 1 : kRow16kLds<HALF>];
   __shared__ float red[ROWS * (T / 64 > 0 ? T / 64 : 1)];
   __shared__ int ired[T / 64];
 
   const int sub = threadIdx.x >> LOGT;
   const int t = threadIdx.x & (T - 1);
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * ROWS + sub;
+  const int64_t row = static_cast<int64_t>(xcd_row_group<ROWS>(blockIdx.x, static_cast<uint32_t>(m))) * ROWS + sub;
   if constexpr (T > 64) {
     if (row >= m) return;  // ROWS == 1: the whole workgroup leaves together
   } else {
     if (row >= m) return;  // the wave owns its row: no workgroup barrier below
   }
-  float* L = lds + sub * LROW;
-
-  float v[R];
   const _Float16* xr = x + row * K + t * R;
+  if constexpr (T > 64) {
+    static_assert(!NORM, "the fused RMSNorm reduces over one wave");
+    row16k_in xv[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) xv[c] = *reinterpret_cast<const row16k_in*>(xr + 8 * c);
+    fwht_quant_row16k<HALF, E3M2>(xv, lds, red, ired, t, row, q, sa, qcorr, inv_sqrt_k);
+    return;
+  }
+  float v[R];
 #pragma unroll
   for (int c = 0; c < R / 8; ++c) {
     const half8 h = *reinterpret_cast<const half8*>(xr + 8 * c);
@@ -215,7 +234,6 @@ __global__ __launch_bounds__(ROWS << LOGT) void fwht_quant_kernel(
     for (int e = 0; e < 8; ++e) v[8 * c + e] = static_cast<float>(h[e]);
   }
   if constexpr (NORM) {
-    static_assert(T == 64, "the fused RMSNorm reduces over one wave");
     // The norm weights are loaded with the row, before the sum of squares needs it.
     half8 wv[R / 8];
 #pragma unroll
@@ -224,13 +242,7 @@ __global__ __launch_bounds__(ROWS << LOGT) void fwht_quant_kernel(
     rms_norm_row_wave<K>(v, wv, eps, unit_offset);
   }
 
-  if constexpr (T == 64) {
-    (void)L;
-    fwht_quant_row_wave<LOGK, E3M2>(v, t, row, q, sa, qcorr, inv_sqrt_k);
-  } else {
-    static_assert(!E3M2, "E3M2 codes come from the one-wave rows");
-    fwht_quant_row<LOGK, LOGT>(v, L, red, ired, t, row, q, sa, qcorr, inv_sqrt_k);
-  }
+  if constexpr (T == 64) fwht_quant_row_wave<LOGK, E3M2>(v, t, row, q, sa, qcorr, inv_sqrt_k);
 }
 
 // Unrotated quantization for every other K (K % 64 == 0): int4_gemm.cu:451-477.
@@ -343,13 +355,22 @@ hipError_t launch_quantize(const void* x, int64_t m, int32_t k, int32_t* q, floa
   const dim3 grid(static_cast<unsigned>(m));
   switch (k) {
     case 16384: {
-      // Cache warming fills the slots that the last round of rows leaves idle (68 KB of LDS
-      // per row: two workgroups per CU).
-      const int64_t kSlots = 2 * static_cast<int64_t>(device_cu_count());
+      // Half-row transposes (36 KB of LDS, 131 VGPRs: three workgroups per CU) beyond four rows
+      // per CU, whole rows (68 KB: two) up to there, where one row's own time counts.  Measured
+      // (whole / half, us): 776 rows 14.8 / 16.0, 1024 16.1 / 17.5, 1552 26.0 / 24.0, 3104
+      // 44.4 / 39.3, 6208 80.3 / 69.6.  Cache warming fills the slots that the last round of
+      // rows leaves idle.
+      const bool half = m > 4 * static_cast<int64_t>(device_cu_count());
+      const int64_t kSlots = (half ? 3 : 2) * static_cast<int64_t>(device_cu_count());
       const int64_t tail = m % kSlots;
       const int64_t extra = (warm != nullptr && warm->nbuf > 0 && tail != 0) ? kSlots - tail : 0;
-      fwht_quant_kernel<14, 8, 1><<<dim3(static_cast<unsigned>(m + extra)), 256, 0, stream>>>(
-          xh, m, q, sa, qcorr, inv_sqrt_k, nullptr, 0.0f, 0, extra > 0 ? *warm : CacheWarmParams{});
+      const dim3 g16(static_cast<unsigned>(m + extra));
+      const CacheWarmParams wp = extra > 0 ? *warm : CacheWarmParams{};
+      if (half)
+        fwht_quant_kernel<14, 8, 1, false, false, true><<<g16, 256, 0, stream>>>(xh, m, q, sa, qcorr, inv_sqrt_k,
+                                                                                 nullptr, 0.0f, 0, wp);
+      else
+        fwht_quant_kernel<14, 8, 1><<<g16, 256, 0, stream>>>(xh, m, q, sa, qcorr, inv_sqrt_k, nullptr, 0.0f, 0, wp);
       break;
     }
     case 2048:
@@ -400,6 +421,11 @@ hipError_t launch_quantize_e3m2(const void* x, const void* nw, float eps, int un
                                 int32_t k, void* q6, float* sa, float inv_sqrt_k, hipStream_t stream,
                                 const CacheWarmParams* warm) {
   if (m <= 0) return hipSuccess;
+  if (k == 16384 && nw == nullptr) {
+    fwht_quant_kernel<14, 8, 1, false, true, true><<<dim3(static_cast<unsigned>(m)), 256, 0, stream>>>(
+        static_cast<const _Float16*>(x), m, static_cast<int32_t*>(q6), sa, nullptr, inv_sqrt_k);
+    return hipGetLastError();
+  }
   if (k != 2048) return hipErrorInvalidValue;
   // Cache warming as in launch_rmsnorm_quantize: one workgroup per CU the rows leave idle.
   const int64_t row_blocks = (m + 3) / 4;

@@ -181,151 +181,6 @@ __device__ __forceinline__ void store_e3m2_slot(const float (&c)[32], int t, int
   *reinterpret_cast<uint2*>(frag + 1024 + 8 * slot) = make_uint2(d[4], d[5]);
 }
 
-// Rotation, quantization and stores of one row of K = 2^LOGK values held by T = 2^LOGT
-// threads, R = K/T consecutive values per thread (thread t: elements t*R .. t*R + R - 1).
-// The log2(K) butterfly stages run in passes of r = log2(R) consecutive stride bits, each
-// pass entirely in registers, with an LDS transpose between passes that re-deals the row
-// so that the next pass's stride bits index a thread's registers.  Stages still run in
-// increasing order of the stride h and each one writes (a + b, a - b), so the rotated
-// values are bit-identical to the CPU transform.  Pass p covers element bits
-// [lo, lo + w): register j of thread t holds element e_p(t, j), whose bits [lo, lo + w)
-// are j mod 2^w and whose other bits, in increasing order, are (t << (r - w)) | (j >> w).
-// After the last pass each thread holds runs of 2^(r - w) >= 8 consecutive elements,
-// which it packs into code words directly.  L: K + 4*(K/R) floats of LDS for this row
-// (4 pad floats per R keep the transposes nearly bank-conflict free); red/ired: T/64
-// floats/ints of LDS when T > 64.  With T == 64 the row belongs to one wave and nothing
-// here waits on other waves.
-template <int LOGK, int LOGT>
-__device__ __forceinline__ void fwht_quant_row(float (&v)[1 << (LOGK - LOGT)], float* L, float* red,
-                                               int* ired, int t, int64_t row, int32_t* __restrict__ q,
-                                               float* __restrict__ sa, int32_t* __restrict__ qcorr,
-                                               float inv_sqrt_k) {
-  constexpr int K = 1 << LOGK;
-  constexpr int T = 1 << LOGT;
-  constexpr int r = LOGK - LOGT;
-  constexpr int R = 1 << r;
-  constexpr int PASSES = (LOGK + r - 1) / r;
-  constexpr int LAST_W = LOGK - (PASSES - 1) * r;
-  static_assert(r >= 3 && r - LAST_W >= 3, "the last pass must leave runs of >= 8 elements");
-  auto addr = [](int e) { return e + 4 * (e >> r); };
-  auto elem = [](int p, int tt, int j) {
-    const int lo = p * r;
-    const int w = (LOGK - lo) < r ? (LOGK - lo) : r;
-    const int rest = (tt << (r - w)) | (j >> w);
-    return (rest & ((1 << lo) - 1)) | ((j & ((1 << w) - 1)) << lo) | ((rest >> lo) << (lo + w));
-  };
-  auto sync = [&]() {
-    if constexpr (T > 64) __syncthreads();
-    else __builtin_amdgcn_wave_barrier();
-  };
-
-#pragma unroll
-  for (int p = 0; p < PASSES; ++p) {
-    if (p > 0) {
-      // Transpose: scatter with the previous pass's mapping, gather with this one's.
-      if (p == 1) {
-#pragma unroll
-        for (int c = 0; c < R / 4; ++c)
-          *reinterpret_cast<float4*>(&L[addr(t * R + 4 * c)]) =
-              make_float4(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
-      } else {
-        // elem(p, t, j) is the OR of disjoint thread bits elem(p, t, 0) and register bits
-        // elem(p, 0, j), and the padded address is linear over such fields, so every
-        // access is one per-thread base plus a compile-time offset (the LDS
-        // instruction's immediate) instead of per-access index arithmetic.
-        float* const wb = L + addr(elem(p - 1, t, 0));
-#pragma unroll
-        for (int j = 0; j < R; ++j) wb[addr(elem(p - 1, 0, j))] = v[j];
-      }
-      sync();
-      const float* const rb = L + addr(elem(p, t, 0));
-#pragma unroll
-      for (int j = 0; j < R; ++j) v[j] = rb[addr(elem(p, 0, j))];
-      sync();
-    }
-    const int w = (LOGK - p * r) < r ? (LOGK - p * r) : r;
-#pragma unroll
-    for (int b = 0; b < r; ++b) {
-      if (b >= w) break;
-#pragma unroll
-      for (int j = 0; j < R; ++j) {
-        if (j & (1 << b)) continue;
-        const float a = v[j], c = v[j + (1 << b)];
-        v[j] = __fadd_rn(a, c);
-        v[j + (1 << b)] = __fsub_rn(a, c);
-      }
-    }
-  }
-
-  float amax = 0.0f;
-#pragma unroll
-  for (int j = 0; j < R; ++j) amax = fmaxf(amax, fabsf(v[j]));
-  amax = wave_max(amax);
-  if constexpr (T > 64) {
-    if ((t & 63) == 0) red[t >> 6] = amax;
-    __syncthreads();
-    amax = red[0];
-#pragma unroll
-    for (int i = 1; i < T / 64; ++i) amax = fmaxf(amax, red[i]);
-  }
-  const float sdiv = __fadd_rn(__fdiv_rn(amax, 7.0f), 1e-12f);
-  if (t == 0) sa[row] = __fmul_rn(sdiv, inv_sqrt_k);
-
-  // Last pass: for each value g of the pass bits the registers j = g + 2^w * i,
-  // i = 0 .. 2^(r-w) - 1, hold consecutive elements; pack them 8 at a time and store two
-  // words (16 codes, 8 bytes: consecutive words of the row's slot in its fragment) at once.
-  constexpr int RUN = R >> LAST_W;
-  constexpr int NW = (1 << LAST_W) * (RUN / 8);  // code words per thread
-  static_assert(RUN % 16 == 0, "runs of 16 codes per 8-byte store");
-  auto gather8 = [&](int g, int u, float (&c8)[8]) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) c8[e] = v[g + (1 << LAST_W) * (8 * u + e)];
-  };
-  uint32_t words[NW];
-  bool tie[NW];
-  bool near_tie = false;
-  const float rcp = __builtin_amdgcn_rcpf(sdiv);
-#pragma unroll
-  for (int g = 0; g < (1 << LAST_W); ++g)
-#pragma unroll
-    for (int u = 0; u < RUN / 8; ++u) {
-      float c8[8];
-      gather8(g, u, c8);
-      const int i = g * (RUN / 8) + u;
-      tie[i] = false;
-      words[i] = quant_pack8_rcp(c8, rcp, tie[i]);
-      near_tie |= tie[i];
-    }
-  if (__builtin_amdgcn_ballot_w64(near_tie) != 0) {  // rare: redo the flagged words exactly
-#pragma unroll
-    for (int g = 0; g < (1 << LAST_W); ++g)
-#pragma unroll
-      for (int u = 0; u < RUN / 8; ++u) {
-        const int i = g * (RUN / 8) + u;
-        if (__builtin_amdgcn_ballot_w64(tie[i]) != 0) {
-          float c8[8];
-          gather8(g, u, c8);
-          const uint32_t exact = quant_pack8(c8, sdiv);
-          words[i] = tie[i] ? exact : words[i];
-        }
-      }
-  }
-#pragma unroll
-  for (int g = 0; g < (1 << LAST_W); ++g)
-#pragma unroll
-    for (int u = 0; u < RUN / 8; u += 2) {
-      const int e0 = elem(PASSES - 1, t, g + (1 << LAST_W) * 8 * u);
-      const uint2 wd = make_uint2(words[g * (RUN / 8) + u], words[g * (RUN / 8) + u + 1]);
-      *reinterpret_cast<uint2*>(&q[frag_word_index(row, e0 >> 3, kblocks128(K))]) = wd;
-    }
-  int s16 = 0;
-#pragma unroll
-  for (int i = 0; i < NW; ++i) s16 += odd_code_sum16(words[i]);
-  s16 = row_sum<T>(s16, ired);  // T == 64: one wave per row, no barrier
-  if (t == 0) qcorr[row] = -8 * s16;
-}
-
-
 // ---- One wave per row, registers only (T = 64).  Lane t holds R = K / 64 consecutive
 // elements t*R .. t*R + R - 1 in v[0..R-1] (r = log2 R register bits, then 6 lane bits).
 // The butterfly stages still run in increasing order of the stride, each writing
@@ -372,6 +227,237 @@ __device__ __forceinline__ void lane_stage(float (&v)[R], int lane) {
     v[j] = __fadd_rn(partner, __uint_as_float(__float_as_uint(v[j]) ^ neg));
   }
 }
+
+// Rotation, quantization and stores of one row of K = 16384 values held by 256 threads,
+// thread t (lane l = t % 64, wave w = t / 64) with the 64 consecutive fp16 values 64 t .. of
+// xv on entry.  The 14 butterfly stages run in increasing order of the stride, each writing
+// (a + b, a - b), in three register passes over element bits 0-5, 6-11 and 12-13, so the
+// rotated values are bit-identical to the CPU transform:
+//   pass 0   registers = bits 0-5, lanes = bits 6-11, waves = bits 12-13.  Its first stage
+//            reads the fp16 pairs directly (v_fma_mix: a * 1 + b, one rounding);
+//   T1       inside a wave, through its own quarter of the LDS: no workgroup barrier;
+//   pass 1   registers = bits 6-11, lanes = bits 0-5;
+//   T2       across the waves;
+//   pass 2   registers = bits 12-13 (2) and 0-3, thread = bits 4-11.
+// Two forms of the transposes:
+//   HALF = false  the whole row at a time (68 KB, two rows per CU): T1 writes and reads a
+//                 wave's 4096 values, T2 writes them back in place, one barrier, and reads.
+//   HALF = true   half a row at a time (36 KB, three rows per CU): v_permlane32_swap exchanges
+//                 bits 5 and 11, then T1 is two 32 x 32 transposes per half wave; T2 takes two
+//                 rounds (bit 11): every wave writes its 32 registers of the round, then the
+//                 two waves that own those elements read them.  Three rows overlap their loads,
+//                 vector work and LDS phases better, but one row takes longer.
+// What bounds it is the chain of one row's phases (load, three register passes of 2 x 64
+// vector instructions per thread and stage pair, two transposes, one wide reduction) and how
+// many rows per CU hide each other's: at 6208 rows 305 MB move in 70 us (4.4 TB/s of the 5.2 a
+// copy reaches; 83 us before with three workgroup-wide transposes and rows written in
+// order); at 776 rows, three rows per CU, 14.8 us (17.0).  With four half rows per CU the
+// compiler has 128 registers and spills: 75.7 us at 6208 rows.
+// L: kRow16kLds<HALF> floats of LDS, padded by 4 floats per 64 (per 32 in T1's half form)
+// against bank conflicts; red / ired: 4 floats / ints.  E3M2: the codes go out as E3M2
+// fragment slots (q points at the q6 buffer; no row corrections).
+template <bool HALF>
+constexpr int kRow16kLds = HALF ? 4 * 2 * 32 * 36 : 256 * 68;
+typedef uint32_t row16k_in __attribute__((ext_vector_type(4)));
+
+template <bool HALF, bool E3M2 = false>
+__device__ __forceinline__ void fwht_quant_row16k(const row16k_in (&xv)[8], float* L, float* red, int* ired, int t,
+                                                  int64_t row, int32_t* __restrict__ q, float* __restrict__ sa,
+                                                  int32_t* __restrict__ qcorr, float inv_sqrt_k) {
+  const int lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  float v[64];
+#pragma unroll
+  for (int i = 0; i < 32; ++i) {  // stage 0: the halves of a dword
+    const uint32_t x = xv[i / 4][i % 4];
+    asm("v_fma_mix_f32 %0, %1, 1.0, %1 op_sel:[0,0,1] op_sel_hi:[1,0,1]" : "=v"(v[2 * i]) : "v"(x));
+    asm("v_fma_mix_f32 %0, %1, 1.0, -%1 op_sel:[0,0,1] op_sel_hi:[1,0,1]" : "=v"(v[2 * i + 1]) : "v"(x));
+  }
+  reg_stage<1>(v);
+  reg_stage<2>(v);
+  reg_stage<3>(v);
+  reg_stage<4>(v);
+  reg_stage<5>(v);
+  if constexpr (HALF) {
+    // After the swap register bit 5 holds element bit 11 and lane bit 5 element bit 5.
+    swap_lane_bit<32, 5>(v);
+    float* const Lw = L + w * (2 * 32 * 36) + (lane >> 5) * (32 * 36);
+    const int l = lane & 31;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+      for (int j = 0; j < 32; j += 4)
+        *reinterpret_cast<float4*>(Lw + l * 36 + j) =
+            make_float4(v[32 * c + j], v[32 * c + j + 1], v[32 * c + j + 2], v[32 * c + j + 3]);
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int j = 0; j < 32; ++j) v[32 * c + j] = Lw[j * 36 + l];
+      __builtin_amdgcn_wave_barrier();
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 64; j += 4)
+      *reinterpret_cast<float4*>(L + t * 68 + j) = make_float4(v[j], v[j + 1], v[j + 2], v[j + 3]);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < 64; ++j) v[j] = L[w * 4352 + lane + 68 * j];
+    __builtin_amdgcn_wave_barrier();
+  }
+  reg_stage<0>(v);
+  reg_stage<1>(v);
+  reg_stage<2>(v);
+  reg_stage<3>(v);
+  reg_stage<4>(v);
+  reg_stage<5>(v);
+  if constexpr (HALF) {
+    // Element e without bit 11 (bits 0-10, then 12-13) of a round at e' + 4 (e' / 64).
+    float u[64];
+    float* const wb = L + w * (2048 + 128) + lane;
+    const float* const rb = L + (t & 127) * 16 + 4 * ((t & 127) >> 2);
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+      for (int j = 0; j < 32; ++j) wb[j * 68] = v[32 * c + j];
+      __syncthreads();
+      if ((w >> 1) == c) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) u[g + 4 * i] = rb[g * (2048 + 128) + i];
+      }
+      if (c == 0) __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < 64; ++j) v[j] = u[j];
+  } else {
+    // Element e at e + 4 (e / 64).
+#pragma unroll
+    for (int j = 0; j < 64; ++j) L[w * 4352 + lane + 68 * j] = v[j];
+    __syncthreads();
+    const float* const rb = L + t * 16 + 4 * (t >> 2);
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) v[g + 4 * i] = rb[g * 4352 + i];
+  }
+  reg_stage<0>(v);
+  reg_stage<1>(v);
+
+  float amax = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 64; ++j) amax = fmaxf(amax, fabsf(v[j]));
+  amax = wave_max(amax);
+  if ((t & 63) == 0) red[t >> 6] = amax;
+  __syncthreads();
+  amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const float sdiv = __fadd_rn(__fdiv_rn(amax, 7.0f), 1e-12f);
+  if (t == 0) sa[row] = __fmul_rn(sdiv, inv_sqrt_k);
+
+  // For each g the registers g + 4 i, i = 0 .. 15, hold the run of 16 consecutive elements from
+  // 16 t + 4096 g on: packed 8 at a time, two words (16 codes, 8 bytes: consecutive words of
+  // the row's slot in its fragment) to a store.
+  constexpr int NW = 8;  // code words per thread
+  auto gather8 = [&](int g, int u, float (&c8)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) c8[e] = v[g + 4 * (8 * u + e)];
+  };
+  bool tie[NW];
+  bool near_tie = false;
+  const float rcp = __builtin_amdgcn_rcpf(sdiv);
+  if constexpr (E3M2) {
+    typedef float v16f __attribute__((ext_vector_type(16)));
+    uint32_t d[2][6];  // runs 2 h and 2 h + 1, three dwords each
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float c[4][8];  // codes + 8
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float c8[8];
+        gather8(2 * h + i / 2, i % 2, c8);
+        tie[i] = false;
+        quant_codes8_rcp(c8, rcp, tie[i], c[i]);
+      }
+      near_tie = tie[0] | tie[1] | tie[2] | tie[3];
+      if (__builtin_amdgcn_ballot_w64(near_tie) != 0) {  // rare: redo the flagged groups exactly
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (__builtin_amdgcn_ballot_w64(tie[i]) != 0) {
+            float c8[8], x8[8];
+            gather8(2 * h + i / 2, i % 2, c8);
+            quant_codes8(c8, sdiv, x8);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) c[i][e] = tie[i] ? x8[e] : c[i][e];
+          }
+        }
+      }
+      v16f ev, od;  // even and odd codes of run 2 h, then of run 2 h + 1
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        ev[i] = c[i / 4][2 * (i & 3)] - 8.0f;
+        od[i] = c[i / 4][2 * (i & 3) + 1] - 8.0f;
+      }
+      const auto x = __builtin_amdgcn_cvt_scalef32_2xpk16_bf6_f32(ev, od, 1.0f);
+#pragma unroll
+      for (int i = 0; i < 6; ++i) d[h][i] = x[i];
+    }
+    // Threads 2u and 2u + 1 hold the two halves of four slots: the even one takes the other's
+    // halves of slots 0 and 1, the odd one of slots 2 and 3, so that a slot is stored whole.
+    const bool odd = (t & 1) != 0;
+    uint32_t mine[6], got[6];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      got[i] = static_cast<uint32_t>(dpp_i<kDppXor1>(static_cast<int>(odd ? d[0][i] : d[1][i])));
+      mine[i] = odd ? d[1][i] : d[0][i];
+    }
+    uint8_t* const q6 = reinterpret_cast<uint8_t*>(q);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      uint32_t w[6];  // the slot's six dwords, the even thread's half first
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        w[i] = odd ? got[3 * h + i] : mine[3 * h + i];
+        w[3 + i] = odd ? mine[3 * h + i] : got[3 * h + i];
+      }
+      const int e0 = 16 * (t & ~1) + 4096 * ((odd ? 2 : 0) + h);  // the slot's first element
+      uint8_t* const frag = q6 + ((row >> 4) * kblocks128(16384) + (e0 >> 7)) * static_cast<int64_t>(kE3m2FragBytes);
+      const int slot = static_cast<int>(row & 15) + 16 * ((e0 >> 5) & 3);
+      *reinterpret_cast<uint4*>(frag + 16 * slot) = make_uint4(w[0], w[1], w[2], w[3]);
+      *reinterpret_cast<uint2*>(frag + 1024 + 8 * slot) = make_uint2(w[4], w[5]);
+    }
+    return;
+  }
+  uint32_t words[NW];
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    float c8[8];
+    gather8(i / 2, i % 2, c8);
+    tie[i] = false;
+    words[i] = quant_pack8_rcp(c8, rcp, tie[i]);
+    near_tie |= tie[i];
+  }
+  if (__builtin_amdgcn_ballot_w64(near_tie) != 0) {  // rare: redo the flagged words exactly
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      if (__builtin_amdgcn_ballot_w64(tie[i]) != 0) {
+        float c8[8];
+        gather8(i / 2, i % 2, c8);
+        const uint32_t exact = quant_pack8(c8, sdiv);
+        words[i] = tie[i] ? exact : words[i];
+      }
+    }
+  }
+  int s16 = 0;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const uint2 wd = make_uint2(words[2 * g], words[2 * g + 1]);
+    *reinterpret_cast<uint2*>(&q[frag_word_index(row, 2 * t + 512 * g, kblocks128(16384))]) = wd;
+    s16 += odd_code_sum16(wd.x) + odd_code_sum16(wd.y);
+  }
+  s16 = row_sum<256>(s16, ired);
+  if (t == 0) qcorr[row] = -8 * s16;
+}
+
 
 // RMSNorm of one row held by one wave (transformers' GemmaRMSNorm, modeling_gemma.py:64-78,
 // weight wv with the (1 + w) offset when unit_offset), in place:

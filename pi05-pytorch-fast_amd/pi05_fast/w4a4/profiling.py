@@ -241,7 +241,7 @@ def _gemm_e3m2_bytes(m: int, k: int, n: int, out_bytes: float) -> float:
 # The kernel classes of the 776-token prefix-LM forward (one decoder layer's launches), as
 # bench.py --only-kernel names them: class -> (kernel name, workgroups, algorithmic bytes,
 # what they are).  gemm_w4a4_kernel<MI, NI, NWAVES, KW, GELU, RING, WPE, QKV_PREP, QFUSE,
-# E3M2, QPRO, NKB>, fwht_quant_kernel<LOGK, LOGT, ROWS, NORM, E3M2>.
+# E3M2, QPRO, NKB>, fwht_quant_kernel<LOGK, LOGT, ROWS, NORM, E3M2, HALF>.
 _M = 776
 TRAFFIC_CLASSES = {
     "gate_up_gelu": ("gemm_w4a4_kernel<7, 4, 4, 1, true, 2, 2, false, false, true, false, 0>", 512,
@@ -268,12 +268,12 @@ TRAFFIC_CLASSES = {
     "o_residual": ("gemm_w4a4_kernel<4, 4, 4, 4, false, 2, 2, false, false, false, false, 4>", 416,
                    _gemm_alg_bytes(_M, 2048, 2048, 2.0 * 2.0 * _M * 2048),
                    "codes A 0.79 MB + weights 2.10 MB + residual 3.18 MB; out 3.18 MB"),
-    "quant_k16384": ("fwht_quant_kernel<14, 8, 1, false, false>", 776, 2.0 * _M * 16384 + _M * 16384 / 2 + 4 * _M,
+    "quant_k16384": ("fwht_quant_kernel<14, 8, 1, false, false, false>", 776, 2.0 * _M * 16384 + _M * 16384 / 2 + 4 * _M,
                      "fp16 x 25.43 MB; codes 6.36 MB + scales"),
-    "rmsnorm_quant_k2048": ("fwht_quant_kernel<11, 6, 4, true, false>", 194,
+    "rmsnorm_quant_k2048": ("fwht_quant_kernel<11, 6, 4, true, false, false>", 194,
                             2.0 * _M * 2048 + 2 * 2048 + _M * 2048 / 2 + 4 * _M,
                             "fp16 x 3.18 MB + norm weight; codes 0.79 MB + scales"),
-    "rmsnorm_quant_e3m2": ("fwht_quant_kernel<11, 6, 4, true, true>", 194,
+    "rmsnorm_quant_e3m2": ("fwht_quant_kernel<11, 6, 4, true, true, false>", 194,
                            2.0 * _M * 2048 + 2 * 2048 + _M * 2048 * 0.75 + 4 * _M,
                            "fp16 x 3.18 MB + norm weight; E3M2 codes 1.19 MB + scales"),
 }
