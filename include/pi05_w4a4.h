@@ -416,8 +416,8 @@ int pi05w4a4_prefix_attention_warm(const void* q, int64_t ld_q, const void* kv_m
  *        three 1 KB chunks; chunk c holds bytes 16c .. 16c+15 of lane L's 48-byte record
  *        [six dwords of column 32p + L%16 | six dwords of column 32p + 16 + L%16] (codes
  *        as in q6) at 16 L.  The N fp32 column scales follow at word N*KB*24.
- * Shapes: K = 2048 for the quantizers (the gate/up input); K % 128 == 0, K <= 2^18 for the
- * GEMM; N % 32 == 0.
+ * Shapes: K = 2048 for the quantizers (the gate/up input), K = 16384 for the one named so (the
+ * down projection's); K % 128 == 0, K <= 2^18 for the GEMM; N % 32 == 0.
  *
  * pi05w4a4_repack_weight_e3m2: an MFMA-layout weight (pi05w4a4_repack_weight's output) ->
  *   w6, not in place (load time).
@@ -428,6 +428,9 @@ int pi05w4a4_prefix_attention_warm(const void* q, int64_t ld_q, const void* kv_m
  * pi05w4a4_gemm_e3m2: gelu_up = 0: pi05w4a4_gemm_multi of 1..3 w6 weights (n[g] columns
  *   into y[g]); gelu_up = 1: pi05w4a4_gemm_gelu_up (ngroups = 2: gate, up with
  *   n[0] == n[1]; y[0] = fp16(gelu_tanh(gate) * up)).  One launch, no workspace.
+ * pi05w4a4_quantize_e3m2_k16384: pi05w4a4_quantize at K = 16384 with the codes written as q6.
+ * pi05w4a4_gemm_e3m2_rows: pi05w4a4_gemm, or with residual_fp16 (may be null)
+ *   pi05w4a4_gemm_residual, on E3M2 operands with tiles for thousands of rows.
  */
 size_t pi05w4a4_q_e3m2_bytes(int64_t m, int32_t k);
 size_t pi05w4a4_e3m2_words(int32_t n, int32_t k);
@@ -441,6 +444,9 @@ int pi05w4a4_rmsnorm_quantize_e3m2_warm(const void* x_fp16, const void* w_fp16, 
 int pi05w4a4_gemm_e3m2(const void* q6, const float* sa, int64_t m, int32_t k, int32_t ngroups,
                        const int32_t* const* w6, const int32_t* n, void* const* y_fp16, int32_t gelu_up,
                        void* stream);
+int pi05w4a4_quantize_e3m2_k16384(const void* x_fp16, int64_t m, void* q6, float* sa, void* stream);
+int pi05w4a4_gemm_e3m2_rows(const void* q6, const float* sa, int64_t m, int32_t k, const int32_t* w6, int32_t n,
+                            const void* residual_fp16, void* y_fp16, void* stream);
 
 #ifdef __cplusplus
 }

@@ -642,6 +642,24 @@ int pi05w4a4_rmsnorm_quantize_e3m2_warm(const void* x_fp16, const void* w_fp16, 
   return quantize_e3m2_call(x_fp16, w_fp16, eps, unit_offset, m, k, q6, sa, stream, &warm);
 }
 
+namespace {
+// Tile counts and modes of the E3M2 main tile (16 mi x 256 outputs; GELU: 128 gate + up) for
+// M rows in ceil(M / 112) equal tiles: the smallest mi >= 4 that covers them (at 200 rows 7,
+// at 130 rows 5).  m-groups of the tile order: equal, at most 16 m-tiles (2.8 MB of codes at
+// K = 2048, which stay in an XCD's 4 MB L2).
+void e3m2_main_tiles(w4a4::GemmParams& p, int64_t ntiles) {
+  const int64_t m7 = cdiv(p.m, 112);
+  p.ntiles = static_cast<int32_t>(ntiles);
+  p.mtiles = static_cast<int32_t>(m7);
+  p.mi = static_cast<int32_t>(std::max<int64_t>(4, cdiv(p.m, 16 * m7)));
+  p.mgroup = static_cast<int32_t>(cdiv(m7, cdiv(m7, 16)));
+  p.ksplit = 1;
+  p.kblocks_per_split = w4a4::kblocks128(p.k);
+  p.mblocks = static_cast<int32_t>(cdiv(p.m, 16));
+  p.mode = w4a4::kEpiFp16;
+}
+}  // namespace
+
 int pi05w4a4_gemm_e3m2(const void* q6, const float* sa, int64_t m, int32_t k, int32_t ngroups,
                        const int32_t* const* w6, const int32_t* n, void* const* y_fp16, int32_t gelu_up,
                        void* stream) {
@@ -663,10 +681,8 @@ int pi05w4a4_gemm_e3m2(const void* q6, const float* sa, int64_t m, int32_t k, in
   if (q6 == nullptr || sa == nullptr) return fail(PI05W4A4_EINVAL, "null activation codes or scales");
   if (!aligned(q6, 16) || !aligned(sa, 4))
     return fail(PI05W4A4_EINVAL, "q6 must be 16-byte aligned, sa 4-byte aligned");
-  // Tiles: the main tile (16 mi x 256 outputs; GELU: 128 gate + up) when 112-row tiles give at
-  // least 1.5 workgroups per CU, else 32 x 128 (the narrow GEMMs: QKV, o).  The main tile's
-  // height is the smallest multiple of 16 rows that covers M in ceil(M / 112) equal tiles (at
-  // 200 rows 112, at 130 rows 80).
+  // Tiles: the main tile when 112-row tiles give at least 1.5 workgroups per CU, else 32 x 128
+  // (the narrow GEMMs: QKV, o).
   const int64_t cus = w4a4::device_cu_count();
   const int64_t m7 = cdiv(m, 112);
   int64_t n7 = 0;
@@ -692,17 +708,50 @@ int pi05w4a4_gemm_e3m2(const void* q6, const float* sa, int64_t m, int32_t k, in
     tile_begin += static_cast<int>(cdiv(n[g], tile_cols));
     n_total += n[g];
   }
-  p.ntiles = gelu_up != 0 ? static_cast<int32_t>(cdiv(n[0], tile_cols)) : tile_begin;
-  p.mtiles = static_cast<int32_t>(mtiles);
-  p.mi = static_cast<int32_t>(std::max<int64_t>(4, cdiv(m, 16 * m7)));
-  p.mgroup = static_cast<int32_t>(cdiv(mtiles, cdiv(mtiles, 16)));  // equal groups of at most 16 (2.8 MB at K = 2048)
-  p.ksplit = 1;
-  p.kblocks_per_split = w4a4::kblocks128(k);
-  p.mblocks = static_cast<int32_t>(cdiv(m, 16));
+  e3m2_main_tiles(p, gelu_up != 0 ? cdiv(n[0], tile_cols) : tile_begin);
+  if (narrow) p.mtiles = static_cast<int32_t>(mtiles);
   p.n_total = static_cast<int32_t>(n_total);
   p.gelu_pair_n = gelu_up != 0 ? n[0] : 0;
   p.mode = gelu_up != 0 ? w4a4::kEpiGeluUp : w4a4::kEpiFp16;
   return hip_status(w4a4::launch_gemm_e3m2(p, tile_cfg, static_cast<hipStream_t>(stream)), "E3M2 gemm launch");
+}
+
+int pi05w4a4_quantize_e3m2_k16384(const void* x_fp16, int64_t m, void* q6, float* sa, void* stream) {
+  if (m < 0) return fail(PI05W4A4_EINVAL, "M must be >= 0, got %lld", (long long)m);
+  if (m == 0) return ok();
+  if (!x_fp16 || !q6 || !sa) return fail(PI05W4A4_EINVAL, "null pointer argument");
+  if (!aligned(x_fp16, 16) || !aligned(q6, 16) || !aligned(sa, 4))
+    return fail(PI05W4A4_EINVAL, "x and q6 must be 16-byte aligned, sa 4-byte aligned");
+  if (m > 0x7fffffffLL) return fail(PI05W4A4_EINVAL, "M too large");
+  return hip_status(w4a4::launch_quantize_e3m2(x_fp16, nullptr, 0.0f, 0, m, 16384, q6, sa,
+                                               static_cast<float>(1.0 / std::sqrt(16384.0)),
+                                               static_cast<hipStream_t>(stream), nullptr),
+                    "E3M2 quantize launch");
+}
+
+int pi05w4a4_gemm_e3m2_rows(const void* q6, const float* sa, int64_t m, int32_t k, const int32_t* w6, int32_t n,
+                            const void* residual_fp16, void* y_fp16, void* stream) {
+  if (m < 0) return fail(PI05W4A4_EINVAL, "M must be >= 0, got %lld", (long long)m);
+  const int rc = validate_e3m2_shape(n, k, "weight");
+  if (rc) return rc;
+  if (w6 == nullptr || !aligned(w6, 16)) return fail(PI05W4A4_EINVAL, "the weight must be non-null and 16-byte aligned");
+  if (m == 0) return ok();
+  if (q6 == nullptr || sa == nullptr || y_fp16 == nullptr)
+    return fail(PI05W4A4_EINVAL, "null activation codes, scales or output");
+  if (!aligned(q6, 16) || !aligned(sa, 4) || !aligned(y_fp16, 16) || !aligned(residual_fp16, 16))
+    return fail(PI05W4A4_EINVAL, "q6, the output and the residual must be 16-byte aligned, sa 4-byte aligned");
+  const int64_t m7 = cdiv(m, 112);
+  if (m7 > 65535) return fail(PI05W4A4_EINVAL, "M too large (%lld rows)", (long long)m);
+  w4a4::GemmParams p{};
+  p.q = static_cast<const int32_t*>(q6);
+  p.sa = sa;
+  p.m = m;
+  p.k = k;
+  p.ngroups = 1;
+  p.g[0] = w4a4::GemmGroup{w6, y_fp16, n, 0};
+  p.res = static_cast<const _Float16*>(residual_fp16);
+  e3m2_main_tiles(p, cdiv(n, 256));
+  return hip_status(w4a4::launch_gemm_e3m2(p, w4a4::kCfg7x4, static_cast<hipStream_t>(stream)), "E3M2 gemm launch");
 }
 
 int pi05w4a4_gemm_gelu_up(const int32_t* q, const float* sa, int64_t m, int32_t k,

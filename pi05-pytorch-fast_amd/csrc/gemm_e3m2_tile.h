@@ -332,9 +332,25 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
   const int8_t* const fix = reinterpret_cast<const int8_t*>(lds + T::kFix);
   char* const yw = reinterpret_cast<char*>(cur.y + m0 * N + wcol);
   const uint32_t loff = static_cast<uint32_t>((lane / LPR) * N + (lane % LPR) * 8) * 2u;
+  // Residual: the 16-byte pieces that this wave's store loop adds, two row blocks ahead
+  // (addresses clamped into the matrix; pieces outside it are never stored).
   const bool has_res = !GELU && p.res != nullptr;
+  uint4 resv[GELU ? 1 : 3][16 / RPI];
+  auto load_res = [&](int mi) {
+    if constexpr (!GELU) {
+      if (mi < MI && has_res) {
+        const _Float16* const rcol = p.res + min(wcol + (lane % LPR) * 8, N - 8);
+#pragma unroll
+        for (int j = 0; j < 16 / RPI; ++j)
+          resv[mi % 3][j] = *reinterpret_cast<const uint4*>(rcol + min(m0 + mi * 16 + j * RPI + lane / LPR, M - 1) * N);
+      }
+    }
+  };
+  load_res(0);
+  load_res(1);
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi) {
+    load_res(mi + 2);
 #pragma unroll
     for (int ni = 0; ni < (GELU ? 2 : NI); ++ni) {
       const float swv[4] = {sw[ni].x, sw[ni].y, sw[ni].z, sw[ni].w};
@@ -371,11 +387,7 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
       char* const yrow = yw + static_cast<int64_t>(mi * 16 + j * RPI) * N * 2;  // uniform; + loff per lane
       if (m0 + trow < M && wcol + tcol < N) {
         if constexpr (!GELU) {
-          if (has_res) {
-            half8 o8 = __builtin_bit_cast(half8, v);
-            o8 += *reinterpret_cast<const half8*>(reinterpret_cast<const char*>(p.res) + (yrow - reinterpret_cast<char*>(cur.y)) + loff);
-            v = __builtin_bit_cast(uint4, o8);
-          }
+          if (has_res) v = __builtin_bit_cast(uint4, __builtin_bit_cast(half8, v) + __builtin_bit_cast(half8, resv[mi % 3][j]));
         }
         __builtin_nontemporal_store(v4i{static_cast<int>(v.x), static_cast<int>(v.y), static_cast<int>(v.z), static_cast<int>(v.w)},
                                     reinterpret_cast<v4i*>(yrow + loff));

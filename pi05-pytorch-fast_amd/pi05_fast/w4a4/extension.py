@@ -142,6 +142,8 @@ def load_int4_gemm():
             ctypes.c_int, [vp, vp, ctypes.c_float, i32, i64, i32, vp, vp, ctypes.POINTER(vp), ctypes.POINTER(sz), i32,
                            vp]),
         "pi05w4a4_gemm_e3m2": (ctypes.c_int, [vp, vp, i64, i32, i32, vp, vp, vp, i32, vp]),
+        "pi05w4a4_quantize_e3m2_k16384": (ctypes.c_int, [vp, i64, vp, vp, vp]),
+        "pi05w4a4_gemm_e3m2_rows": (ctypes.c_int, [vp, vp, i64, i32, vp, i32, vp, vp, vp]),
     }
     for name, (res, args) in sig.items():
         fn = getattr(lib, name)
@@ -504,6 +506,40 @@ def int4_twin(w: torch.Tensor, k: int) -> torch.Tensor | None:
     return twin
 
 
+# E3M2 forms of INT4 MFMA-layout K = 16384 weights (the down projection), registered by the
+# loader: calls of at least E3M2_MIN_ROWS_K16384 rows run on them.  The INT4 kernel's 112 x 64
+# tiles of eight K-split waves take a CU each: 1792 rows of N = 2048 are two full rounds of 256
+# CUs, and every further 896 rows a round more, while the E3M2 tile's 112 x 256 tiles pay one
+# workgroup time up to 3584 rows.  Measured (activation quant + GEMM + residual, us, INT4 /
+# E3M2): 1500 rows 83 / 92, 1792 86 / 96, 1793 98 / 96, 2128 107 / 101, 2688 134 / 107, 3584
+# 189 / 121, 4480 235 / 170, 6208 243 / 222.  An entry lives as long as its INT4 weight and is
+# ignored once that weight is modified in place, like a twin's.
+E3M2_MIN_ROWS_K16384 = 1793
+_E3M2_FORMS: dict[int, tuple] = {}
+
+
+def register_e3m2_form(w_int4: torch.Tensor, w_e3m2: torch.Tensor, k: int) -> None:
+    """Record w_e3m2 as the E3M2 form of the MFMA-layout weight w_int4."""
+    if not (is_e3m2_layout(w_e3m2, k) and is_mfma_layout(w_int4, k)):
+        raise RuntimeError("register_e3m2_form takes an MFMA-layout weight and its E3M2-layout form")
+    if int(w_e3m2.size(0)) != int(w_int4.size(0)):
+        raise RuntimeError("the two forms of a weight must have the same N")
+    key = id(w_int4)
+    _E3M2_FORMS[key] = (weakref.ref(w_int4, lambda _r, key=key: _E3M2_FORMS.pop(key, None)), w_int4._version,
+                        w_int4.data_ptr(), k, w_e3m2)
+
+
+def e3m2_form(w: torch.Tensor, k: int) -> torch.Tensor | None:
+    """The registered E3M2 form of the MFMA-layout weight w, or None."""
+    hit = _E3M2_FORMS.get(id(w))
+    if hit is None:
+        return None
+    ref, version, ptr, hk, form = hit
+    if ref() is not w or version != w._version or ptr != w.data_ptr() or hk != k:
+        return None
+    return form
+
+
 def gemm_weights_for_rows(ws: list[torch.Tensor], k: int, m: int) -> list[torch.Tensor]:
     """The tensors a call of m rows on the weights ws reads: the INT4 twins of E3M2-layout
     weights at m <= E3M2_MAX_INT4_ROWS when every weight has one, else ws (for cache
@@ -517,13 +553,14 @@ def gemm_weights_for_rows(ws: list[torch.Tensor], k: int, m: int) -> list[torch.
 
 def clear_weight_caches() -> None:
     """Drop every derived copy of a weight that the ops keep (the repacked L1/L2/L3
-    weights, the RoPE-pair K weights of fused decoder layers and the INT4 twins of E3M2
-    weights), so that the next call rebuilds them from the current weights (a twin is not
-    rebuilt: calls on its E3M2 weight run the E3M2 kernels).  Needed after writing a
-    weight in place through ``.data`` (which bypasses the version counter the caches
-    check)."""
+    weights, the RoPE-pair K weights of fused decoder layers, the INT4 twins of E3M2 weights
+    and the E3M2 forms of K = 16384 weights), so that the next call rebuilds them from the
+    current weights (twins and forms are not rebuilt: calls run on the weight given).
+    Needed after writing a weight in place through ``.data`` (which bypasses the version
+    counter the caches check)."""
     _MFMA_CACHE.clear()
     _INT4_TWINS.clear()
+    _E3M2_FORMS.clear()
     for fn in _CACHE_CLEARERS:
         fn()
 
@@ -812,6 +849,10 @@ def _run(x: torch.Tensor, ws: list[torch.Tensor], tiled: bool, kind: str, gelu: 
     if residual is not None:  # before any launch: the kernel reads it through a raw pointer
         _check_residual(residual, x.device, (*x.shape[:-1], int(ws[0].size(0))))
     m = x.numel() // k
+    if k == 16384 and m >= E3M2_MIN_ROWS_K16384 and len(ws) == 1 and norm is None and not tiled:
+        form = e3m2_form(ws[0], k)
+        if form is not None and form.device == x.device:
+            return _run_e3m2_rows(x, form, k, m, residual)
     if not gelu and k == 2048 and 1 <= m <= SMALL_M_MAX_ROWS and x.is_cuda:
         return _run_small(x, ws, k, m, tiled, kind, norm, residual)
     # the reference quantizes before checking the weights
@@ -888,6 +929,29 @@ def _run_e3m2(x, ws, k, n_e3m2, kind, gelu, norm, residual, warm=None):
     dev = x.device
     with _on_device(dev):
         return _gemm_e3m2_from_q(q6, sa, k, ws, tuple(x.shape[:-1]), dev, gelu=gelu)
+
+
+def _run_e3m2_rows(x, w6, k, m, residual):
+    """_run for one K = 16384 weight at thousands of rows, on its E3M2 form w6."""
+    x2 = x if x.is_contiguous() else x.contiguous()
+    if x2.data_ptr() % 16:
+        x2 = x2.clone()
+    lib = _lib if _lib is not None else load_int4_gemm()
+    dev = x2.device
+    n = int(w6.size(0))
+    res = None
+    if residual is not None:
+        res = residual if residual.is_contiguous() and residual.data_ptr() % 16 == 0 else residual.contiguous().clone()
+    q6 = torch.empty((_q6_bytes(m, k),), dtype=torch.uint8, device=dev)
+    sa = torch.empty((m,), dtype=torch.float32, device=dev)
+    out = torch.empty((m, n), dtype=torch.float16, device=dev)
+    with _on_device(dev):
+        st = _stream(dev)
+        _check(lib.pi05w4a4_quantize_e3m2_k16384(x2.data_ptr(), m, q6.data_ptr(), sa.data_ptr(), st),
+               "pi05w4a4_quantize_e3m2_k16384")
+        _check(lib.pi05w4a4_gemm_e3m2_rows(q6.data_ptr(), sa.data_ptr(), m, k, w6.data_ptr(), n, _ptr(res),
+                                           out.data_ptr(), st), "pi05w4a4_gemm_e3m2_rows")
+    return [out.view(*x.shape[:-1], n)]
 
 
 def _rms_norm_impl(x: torch.Tensor, weight: torch.Tensor, eps: float, unit_offset: bool) -> torch.Tensor:
