@@ -555,7 +555,7 @@ _KERNEL_CLASS_RULES = (
     (r"fwht_quant_kernel(?:<14,|ILi14E)", "quant_k16384"),
     (r"fwht_quant_kernel(?:<11, 6, 4, true[,>]|ILi11ELi6ELi4ELb1E)", "rmsnorm_quant_k2048"),
     (r"fwht_quant_kernel(?:<11,|ILi11E)", "quant_k2048"),
-    (r"prefix_attention_kernel", "attention"),
+    (r"prefix_attention_(?:wide_)?kernel", "attention"),
     (r"kv_prep_kernel", "attn_kv_prep"),
     (r"rmsnorm_kernel", "rmsnorm"),
 )

@@ -26,8 +26,9 @@
 // 16-byte operands of one MFMA, so every operand fetch below is one contiguous 1 KB
 // wave load.  K fragment (j, t): lane L = K[16j + L%16][32t + 8(L/16) + 0..7];
 // V^T fragment (db, t): lane L = V[32t + 8(L/16) + 0..7][16db + L%16].
-// One workgroup (8 waves) owns 32 consecutive rows (4 tokens x 8 heads for PaliGemma)
-// and every key of its KV head:
+// Launches of three and more rounds of these workgroups run attention_wide.h's kernel
+// instead.  One workgroup (8 waves) owns 32 consecutive rows (4 tokens x 8 heads for
+// PaliGemma) and every key of its KV head:
 //   phase 0  the 32 query rows are loaded once, RoPE'd and stored to LDS; each wave then
 //            reads them as MFMA operands;
 //   phase 1  S^T = K Q^T with v_mfma_f32_16x16x32_f16, the waves taking 16-key blocks in
@@ -470,6 +471,11 @@ __global__ __launch_bounds__(kThreads) void prefix_attention_kernel(const AttnPa
 }
 
 }  // namespace
+}  // namespace w4a4
+
+#include "attention_wide.h"
+
+namespace w4a4 {
 
 int64_t attn_s_pad(int32_t s) { return (static_cast<int64_t>(s) + 63) / 64 * 64; }
 
@@ -480,14 +486,44 @@ hipError_t launch_attn_kv_prep(const AttnParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// The 128-row kernel from the third round of 32-row workgroups on (one per CU).  Its rounds
+// hold two workgroups per CU: up to one workgroup per CU they take as long as 2-3 rounds of
+// the 32-row kernel, up to two as 3-4, and the 32-row kernel's last round is often nearly
+// empty.  us with the K/V prep, 32-row / 128-row workgroups (tokens x batch, masked; 32-row
+// rounds): 776 x 2 (1.5) 34.8 / 39.1, 1024 x 2 (2.0) 42.8 / 47.0, 389 x 4 (1.5) 30.9 / 31.2,
+// 389 x 5 (1.9) 33.0 / 32.3; 776 x 3 (2.3) 50.1 / 40.7, 389 x 6 (2.3) 41.9 / 33.8, 100 x 24
+// (2.3) 25.4 / 18.2, 8 x 300 (2.3) 30.9 / 20.9, 1 x 600 (2.3) 37.8 / 31.8, 776 x 6 (4.5) 74.9 /
+// 59.5, 776 x 8 (6.1) 99.9 / 62.2, 1024 x 8 (8.0) 138 / 83.
+// It scales the scores with packed fp16 products, the same bits where the scaling is itself
+// an fp16 number, and holds a sequence's mask offsets in 32 bits.
+static bool takes_wide(const AttnParams& p, int64_t rows, int64_t cus) {
+  const int64_t groups = static_cast<int64_t>(p.kvh) * p.b;
+  const int64_t wgs32 = (rows + kRows - 1) / kRows * groups;
+  if (wgs32 <= 2 * cus || wgs32 >= (int64_t{1} << 30)) return false;
+  if (static_cast<float>(static_cast<_Float16>(p.scaling)) != p.scaling) return false;  // also NaN
+  if (p.mask != nullptr && p.mask_rs > ((int64_t{1} << 30) - p.mask_len) / p.s) return false;
+  return true;
+}
+
 hipError_t launch_prefix_attention(const AttnParams& p_in, hipStream_t stream) {
   AttnParams p = p_in;
   const int64_t rows = static_cast<int64_t>(p.s) * (p.h / p.kvh);
+  const int64_t kCUs = device_cu_count();
+  if (takes_wide(p, rows, kCUs)) {
+    p.row_blocks = static_cast<int32_t>((rows + kWideRows - 1) / kWideRows);
+    const int64_t wgs = static_cast<int64_t>(p.row_blocks) * p.kvh * p.b;
+    const unsigned grid = static_cast<unsigned>(8 * ((wgs + 7) / 8));
+    const size_t lds = p.qcodes != nullptr ? kWideLdsQuant : kWideLds;
+    if (p.mask != nullptr)
+      prefix_attention_wide_kernel<true><<<grid, kWideThreads, lds, stream>>>(p);
+    else
+      prefix_attention_wide_kernel<false><<<grid, kWideThreads, lds, stream>>>(p);
+    return hipGetLastError();
+  }
   p.row_blocks = static_cast<int32_t>((rows + kRows - 1) / kRows);
   // Cache warming uses the CUs that the attention leaves idle (one workgroup of 8 waves
   // per CU: at ~200 VGPRs a SIMD holds two of its waves, while its ~71 KB of LDS would
   // allow two workgroups): none when the attention alone fills the device's CUs.
-  const int64_t kCUs = device_cu_count();
   const int64_t attn_wgs = static_cast<int64_t>(p.row_blocks) * p.kvh * p.b;
   const int64_t warm_x = (p.warm.nbuf > 0 && attn_wgs < kCUs) ? (kCUs - attn_wgs) / (static_cast<int64_t>(p.kvh) * p.b) : 0;
   const dim3 grid(static_cast<unsigned>(p.row_blocks + warm_x), static_cast<unsigned>(p.kvh),
