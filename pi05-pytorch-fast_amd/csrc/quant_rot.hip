@@ -245,8 +245,72 @@ __global__ __launch_bounds__(ROWS << LOGT, HALF ? 3 : 1) void fwht_quant_kernel(
   if constexpr (T == 64) fwht_quant_row_wave<LOGK, E3M2>(v, t, row, q, sa, qcorr, inv_sqrt_k);
 }
 
-// Unrotated quantization for every other K (K % 64 == 0): int4_gemm.cu:451-477.
-// One workgroup of 256 threads per row, two passes over the row (amax, then codes).
+// Unrotated quantization for every other K (K % 64 == 0), int4_gemm.cu:451-477, up to
+// K = 1024 * PAIRS: one wave per row, the row in registers, lane t the 16-code pairs of words
+// t + 64 i, the codes through quant_pack8_rcp (exact division only near ties).  Four rows per
+// workgroup; the workgroups of a 16-row block, whose code words share 128-byte lines, run on
+// one XCD (workgroup i runs on XCD i % 8) as far as whole groups of 128 rows go.
+// What bounds it: latency (a row is read once, one wave-wide max, one sum) and, at thousands
+// of rows, the vector instructions of the codes.  us in a graph, a workgroup per row / this:
+// K = 512: 200 rows 2.88 / 2.64, 1000 3.21 / 2.91, 6208 8.24 / 4.69; K = 4096: 1 row 3.11 /
+// 3.32, 200 3.77 / 3.87, 1000 6.54 / 4.26, 6208 24.3 / 13.5; K = 8192: 200 5.25 / 5.39, 1000
+// 10.6 / 6.3, 6208 49.4 / 25.8.  So beyond K = 1024 a few rows, whose time is one row's
+// latency, keep a workgroup each (K = 1536 to 8192: up to 0.9 us faster at 200 rows, 0.85 to
+// 4.3 us slower at 1000).
+constexpr int64_t kWaveRowsMin = 512;
+template <int PAIRS>
+__global__ __launch_bounds__(256) void quant_rows_wave_kernel(const _Float16* __restrict__ x, int64_t m, int32_t k,
+                                                              int32_t* __restrict__ q, float* __restrict__ sa,
+                                                              int32_t* __restrict__ qcorr) {
+  const int64_t row = 4 * static_cast<int64_t>(xcd_row_group<4>(blockIdx.x, static_cast<uint32_t>(m))) + (threadIdx.x >> 6);
+  if (row >= m) return;  // a whole wave
+  const int t = threadIdx.x & 63;
+  const int pairs = k / 16;
+  const _Float16* xr = x + row * k;
+  half8 h[PAIRS][2];
+#pragma unroll
+  for (int i = 0; i < PAIRS; ++i) {
+    const int c = t + 64 * i;
+    h[i][0] = h[i][1] = half8{};
+    if (c < pairs) {
+      h[i][0] = *reinterpret_cast<const half8*>(xr + 16 * c);
+      h[i][1] = *reinterpret_cast<const half8*>(xr + 16 * c + 8);
+    }
+  }
+  float amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < PAIRS; ++i)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) amax = fmaxf(amax, fabsf(static_cast<float>(h[i][j >> 3][j & 7])));
+  amax = wave_max_dpp(amax);
+  const float sdiv = __fadd_rn(__fdiv_rn(amax, 7.0f), 1e-12f);
+  if (t == 0) sa[row] = sdiv;
+  const float rcp = __builtin_amdgcn_rcpf(sdiv);
+  const int32_t kb = kblocks128(k);
+  int s16 = 0;
+#pragma unroll
+  for (int i = 0; i < PAIRS; ++i) {
+    const int c = t + 64 * i;
+    uint32_t w[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = static_cast<float>(h[i][u][e]);
+      bool near_tie = false;
+      w[u] = quant_pack8_rcp(v, rcp, near_tie);
+      if (near_tie) w[u] = quant_pack8(v, sdiv);
+    }
+    if (c < pairs) {
+      *reinterpret_cast<uint2*>(&q[frag_word_index(row, 2 * c, kb)]) = make_uint2(w[0], w[1]);
+      s16 += odd_code_sum16(w[0]) + odd_code_sum16(w[1]);
+    }
+  }
+  s16 = wave_sum_dpp(s16);
+  if (t == 0) qcorr[row] = -8 * s16;
+}
+
+// Longer rows, and few of them beyond K = 1024: one workgroup of 256 threads per row, two passes over the row (amax, then codes).
 __global__ __launch_bounds__(256) void quant_rows_kernel(const _Float16* __restrict__ x, int64_t m,
                                                          int32_t k, int32_t* __restrict__ q,
                                                          float* __restrict__ sa,
@@ -385,9 +449,20 @@ hipError_t launch_quantize(const void* x, int64_t m, int32_t k, int32_t* q, floa
     case 1024:
       quant_rot_kernel<1024, 128><<<grid, 128, 0, stream>>>(xh, m, q, sa, qcorr, inv_sqrt_k);
       break;
-    default:
-      quant_rows_kernel<<<grid, 256, 0, stream>>>(xh, m, k, q, sa, qcorr);
+    default: {
+      const dim3 g4(static_cast<unsigned>((m + 3) / 4));
+      if (k > 8192 || (k > 1024 && m < kWaveRowsMin))
+        quant_rows_kernel<<<grid, 256, 0, stream>>>(xh, m, k, q, sa, qcorr);
+      else if (k <= 1024)
+        quant_rows_wave_kernel<1><<<g4, 256, 0, stream>>>(xh, m, k, q, sa, qcorr);
+      else if (k <= 2048)
+        quant_rows_wave_kernel<2><<<g4, 256, 0, stream>>>(xh, m, k, q, sa, qcorr);
+      else if (k <= 4096)
+        quant_rows_wave_kernel<4><<<g4, 256, 0, stream>>>(xh, m, k, q, sa, qcorr);
+      else
+        quant_rows_wave_kernel<8><<<g4, 256, 0, stream>>>(xh, m, k, q, sa, qcorr);
       break;
+    }
   }
   return hipGetLastError();
 }

@@ -68,3 +68,23 @@ def test_half_row_form_ties(ext, cuda):
     x = inp.activations(inp.generator(7600), m, k)
     x[m - 16 :] = torch.from_numpy(x16)
     _check(ext, x, cuda, m, k)
+
+
+@pytest.mark.parametrize("m", [1, 3, 127, 129, 511, 512, 513])
+@pytest.mark.parametrize("k", [64, 960, 1088, 4096, 4160, 8192, 8256])
+def test_unrotated_rows_match_oracle(ext, cuda, m, k):
+    """The unrotated quantizer at the edges of its wave-per-row forms (K = 1024, 2048, 4096,
+    8192; 512 rows; runs of 128 rows), with rows whose codes are exact ties:
+    the codes and row sums of every form are the oracle's."""
+    from pi05_fast.w4a4.pack import codes_from_fragment_major, qcorr_from_fragment_major
+
+    gen = inp.generator(31 * k + m)
+    x = _edge_rows(gen, m, k)
+    ties = (torch.randint(-7, 7, x[4::7].shape, generator=gen).float() + 0.5).half()
+    ties[:, 5] = 7.0  # the row's scale is 1: every other value lies between two codes
+    x[4::7] = ties
+    _check(ext, x, cuda, m, k)
+    q, _ = ext.quantize(x.to(cuda))
+    codes = orc.unpack_nibbles(inp.to_np(codes_from_fragment_major(q.cpu(), m, k)), k)
+    want = -128 * codes[:, 1::2].astype(np.int64).sum(axis=1)
+    assert np.array_equal(inp.to_np(qcorr_from_fragment_major(q.cpu(), m, k)), want)
