@@ -33,6 +33,7 @@
 // order; the epilogue's arithmetic is gemm_w4a4_kernel's.
 #pragma once
 
+#include "direct_load.h"
 #include "gelu_tanh.h"
 #include "w4a4_internal.h"
 
@@ -54,20 +55,6 @@ struct E3m2Tile {
   static constexpr int kOut = kFix + (GELU ? kGeluFixEntries : 0);
   static constexpr int kLds = kOut + kWaves * 16 * LSR * 2;
 };
-
-// s_waitcnt vmcnt(N) as asm: it has to count the asm loads, which the compiler does not.
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-__device__ __forceinline__ void lds_done_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// One 1 KB piece from global memory (uniform base + per-lane byte offset) to LDS address
-// `dst` (lane L writes bytes 16 L ..).
-__device__ __forceinline__ void load_lds_1k(const char* base, uint32_t voff, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               ::"v"(voff), "s"(base), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory");
-}
 
 template <int MI, bool GELU>
 __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const int8_t* fix_table) {
@@ -169,9 +156,9 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
   // exact: the last tile's read its own first blocks again.
   v12i b0[2], b1[2];
   auto issue_b = [&](int kb, int qd, v12i (&b)[2]) {
-    const v4i c0 = *reinterpret_cast<const v4i*>(bp[qd] + boff);
-    const v4i c1 = *reinterpret_cast<const v4i*>(bp[qd] + boff + 1024);
-    const v4i c2 = *reinterpret_cast<const v4i*>(bp[qd] + boff + 2048);
+    const v4i c0 = load_16(bp[qd] + boff);
+    const v4i c1 = load_16(bp[qd] + boff + 1024);
+    const v4i c2 = load_16(bp[qd] + boff + 2048);
     const v8i c01 = __builtin_shufflevector(c0, c1, 0, 1, 2, 3, 4, 5, 6, 7);
     const v8i c2x = __builtin_shufflevector(c2, c2, 0, 1, 2, 3, 4, 5, 6, 7);
     b[qd] = __builtin_shufflevector(c01, c2x, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11);
@@ -212,7 +199,8 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
         acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bfrag(b, ni), aop[mi], acc[mi][ni], 3, 3, 0, 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
     issue_b(kb + 2, 0, b);
-    // Younger loads than A stage kb + 1's: four column pairs and A stage kb + 2.
+    // Younger loads than A stage kb + 1's (issued in step kb - 2 or the prologue): pair 1 of block
+    // kb, both pairs of block kb + 1, pair 0 of block kb + 2, three loads each, and A stage kb + 2.
     if (more || kb + 2 < nkb) {
       if (T::kChunks % T::kWaves == 0 || wave < T::kChunks % T::kWaves) wait_vm<12 + T::kPerWave>();
       else wait_vm<12 + T::kPerWave - 1>();
@@ -245,8 +233,10 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
     wr = next_slot(wr);
   };
 
-  // ---- prologue: the correction table; A stages 0-2 and B blocks 0 and 1 of the first tile,
-  // in the loop's order
+  // ---- prologue: A stages 0-2 and B blocks 0 and 1 of the first tile in the order in which the
+  // steps issue them (step kb: pair 0 of block kb + 2, A stage kb + 3, pair 1 of block kb + 2), so
+  // that the steps' counts hold from the first one on: A 0, B 0.0, A 1, B 0.1, B 1.0, A 2, B 1.1;
+  // then the correction table, which no count relies on.
   Tile cur = tile_at(t_next);
   a_start(cur, abase, voff);
 #pragma unroll
@@ -258,14 +248,12 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
       for (int j = 0; j < T::kPerWave; ++j) issue_a(j, s * T::kStage);
       abase += kE3m2FragBytes;
     }
-    if (s == 0) {
-      issue_b(0, 0, b0);
-      issue_b(0, 1, b0);
-    }
+    if (s == 0) issue_b(0, 0, b0);
     if (s == 1) {
+      issue_b(0, 1, b0);
       issue_b(1, 0, b1);
-      issue_b(1, 1, b1);
     }
+    if (s == 2) issue_b(1, 1, b1);
   }
   if constexpr (GELU) {  // its two halves by direct loads, zeros between
     constexpr int kFixPieces = kGeluFixPosPieces + (kGeluFixEntries / 1024 - kGeluFixNegPiece0);
@@ -277,8 +265,8 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
     for (int i = kGeluFixPosPieces * 1024 + tid * 16; i < kGeluFixNegPiece0 * 1024; i += 64 * T::kWaves * 16)
       *reinterpret_cast<int4*>(lds + T::kFix + i) = int4{0, 0, 0, 0};
   }
-  // Stage 0: all but the 12 B loads, (with three stages) the 2 kPerWave or fewer A pieces and
-  // the table pieces after it.
+  // A stage 0: younger are the 12 B loads and (with three stages) A stages 1 and 2, at least
+  // kPerWave - 1 pieces each.
   if (nkb >= 3) wait_vm<12 + 2 * (T::kPerWave - 1)>();
   else wait_vm<12>();
   lds_done_barrier();

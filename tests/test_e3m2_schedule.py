@@ -1,0 +1,42 @@
+"""How the E3M2 GEMM's main tile orders its operands: csrc/gemm_e3m2_tile.h compiled for the CPU
+with stand-ins for its loads, waits and barriers (tests/host/e3m2_tile), at every tile height,
+plain and GELU, short k ranges and walks over several tiles.  A row operand that a wave's own
+counted waits and the barriers do not cover is an error there, while on the GPU it only shows
+when a load happens to be late."""
+
+from __future__ import annotations
+
+import os
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+CSRC = ROOT / "pi05-pytorch-fast_amd" / "csrc"
+
+
+def _emulate(tmp_path: Path, *flags: str) -> subprocess.CompletedProcess:
+    for f in (ROOT / "tests" / "host" / "e3m2_tile").iterdir():
+        shutil.copy(f, tmp_path)
+    shutil.copy(CSRC / "gemm_e3m2_tile.h", tmp_path)  # beside the stand-ins, which its includes then find
+    rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+    exe = tmp_path / "emulate"
+    subprocess.run([str(rocm / "llvm" / "bin" / "clang++"), "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__",
+                    f"-I{rocm / 'include'}", f"-I{CSRC}", *flags, str(tmp_path / "emulate.cpp"), "-o", str(exe)],
+                   check=True, capture_output=True, text=True)
+    return subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+
+
+def test_every_row_operand_is_covered_by_the_counted_waits(tmp_path):
+    run = _emulate(tmp_path)
+    assert run.returncode == 0, run.stdout[-3000:]
+
+
+@pytest.mark.parametrize("loose", [1, 3])
+def test_the_emulation_notices_a_count_that_is_too_large(tmp_path, loose):
+    run = _emulate(tmp_path, f"-DEMULATE_LOOSE={loose}")
+    for mi in (4, 5, 6, 7):
+        for form in ("plain", "GELU"):
+            assert f"MI {mi} {form}, 16 k blocks" in run.stdout

@@ -1,6 +1,7 @@
-"""The E3M2 GEMM's main tile at its edges: every tile height, ragged rows and columns, the
-shortest k ranges (one to five 128-deep blocks, odd counts among them) and grids in which a
-workgroup walks several tiles, against exact integer arithmetic on the same codes."""
+"""The E3M2 GEMM's main tile at its edges: every tile height (plain, paired and with a
+residual), ragged rows and columns, the shortest k ranges (one to five 128-deep blocks, odd
+counts among them) and grids in which a workgroup walks several tiles, against exact integer
+arithmetic on the same codes."""
 
 from __future__ import annotations
 
@@ -73,7 +74,10 @@ def test_gelu_pairs(ext, cuda, m, k, n):
     assert torch.equal(y.view(torch.int16), ext.gelu_tanh_mul(*want).view(torch.int16))
 
 
-@pytest.mark.parametrize("m,k,n", [(128, 128, 40960), (300, 384, 24608), (784, 512, 16384), (2240, 2048, 4096)])
+# tile heights 64, 80, 80, 96, 96, 64, 112, 112, 112, 112 rows
+@pytest.mark.parametrize("m,k,n", [(64, 512, 90144), (225, 256, 24608), (240, 2048, 24608), (241, 384, 24608),
+                                   (288, 512, 24608), (128, 128, 40960), (300, 384, 24608), (784, 512, 16384),
+                                   (2240, 2048, 4096), (336, 256, 24608)])
 def test_plain_groups(ext, cuda, m, k, n):
     """Two weights of different widths whose 112-row tiles fill the device (the main tile)."""
     gen = inp.generator(9500 + m + k)
@@ -88,3 +92,25 @@ def test_plain_groups(ext, cuda, m, k, n):
         b = torch.from_numpy(orc.unpack_nibbles(inp.to_np(w[:, : k // 8]), k).astype(np.float32)).to(cuda)
         want = (((codes.float() @ b.t()) * sa[:, None]) * w[:, k // 8].view(torch.float32)[None]).half()
         assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
+# tile heights 64, 80, 96 and 112 rows on odd and even counts of k blocks; then (the last two) more
+# tiles than two per CU, so that a workgroup goes on to a second tile past its epilogue
+@pytest.mark.parametrize("m,k,n", [(64, 256, 288), (70, 384, 2080), (96, 2048, 288), (200, 640, 96), (1000, 512, 16416),
+                                   (1500, 1024, 16384)])
+def test_rows_with_residual(ext, cuda, m, k, n):
+    gen = inp.generator(9800 + m + k)
+    codes = torch.randint(-7, 8, (m, k), generator=gen, dtype=torch.int32).to(cuda)
+    sa = (torch.rand(m, generator=gen) * 0.02 + 0.001).to(cuda)
+    packed = inp.random_packed(gen, n, k).to(cuda)
+    w6 = ext.repack_weight_e3m2(packed, k=k)
+    res = torch.randn(m, n, generator=gen).half().to(cuda)
+    q6 = _q6(codes)
+    b = torch.from_numpy(orc.unpack_nibbles(inp.to_np(packed[:, : k // 8]), k).astype(np.float32)).to(cuda)
+    want = (((codes.float() @ b.t()) * sa[:, None]) * packed[:, k // 8].view(torch.float32)[None]).half()
+    for r, ref in ((None, want), (res, want + res)):
+        y = torch.full((m, n), float("nan"), dtype=torch.float16, device=cuda)
+        ext._check(ext.load_int4_gemm().pi05w4a4_gemm_e3m2_rows(
+            q6.data_ptr(), sa.data_ptr(), m, k, w6.data_ptr(), n, ext._ptr(r), y.data_ptr(), ext._stream(sa.device)),
+            "pi05w4a4_gemm_e3m2_rows")
+        assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
