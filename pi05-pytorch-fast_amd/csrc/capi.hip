@@ -651,8 +651,8 @@ void e3m2_main_tiles(w4a4::GemmParams& p, int64_t ntiles) {
   const int64_t m7 = cdiv(p.m, 112);
   p.ntiles = static_cast<int32_t>(ntiles);
   p.mtiles = static_cast<int32_t>(m7);
-  p.mi = static_cast<int32_t>(std::max<int64_t>(4, cdiv(p.m, 16 * m7)));
-  p.mgroup = static_cast<int32_t>(cdiv(m7, cdiv(m7, 16)));
+  p.mi = static_cast<int16_t>(std::max<int64_t>(4, cdiv(p.m, 16 * m7)));
+  p.mgroup = static_cast<int16_t>(cdiv(m7, cdiv(m7, 16)));
   p.ksplit = 1;
   p.kblocks_per_split = w4a4::kblocks128(p.k);
   p.mblocks = static_cast<int32_t>(cdiv(p.m, 16));

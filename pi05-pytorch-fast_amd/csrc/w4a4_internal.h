@@ -45,8 +45,6 @@ struct GemmParams {
   GemmGroup g[kMaxGroups];
   int32_t ntiles;     // total n-tiles over the groups
   int32_t mtiles;
-  int32_t mi;         // E3M2 main tile: row fragments per wave (the tile has 16 mi rows)
-  int32_t mgroup;     // E3M2 main tile: m-tiles per group of the tile order
   int32_t ksplit;     // number of K slices
   int32_t kblocks_per_split;  // 128-deep k blocks per K slice
   int32_t mode;
@@ -89,7 +87,11 @@ struct GemmParams {
   float eps_pro;
   int32_t unit_offset_pro;
   float inv_sqrt_k_pro;
+  int16_t mi;      // E3M2 main tile: row fragments per wave (the tile has 16 mi rows)
+  int16_t mgroup;  // E3M2 main tile: m-tiles per group of the tile order
 };
+// Every GEMM launch copies this block; the last two fields fill its padding.
+static_assert(sizeof(GemmParams) == 352, "kernel arguments of the GEMMs");
 constexpr int kQproMaxRows = 4;
 
 // Control block of the fused gate/up + down-quant launch, in 128-byte lines so that the

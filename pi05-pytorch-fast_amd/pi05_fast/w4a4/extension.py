@@ -849,12 +849,12 @@ def _run(x: torch.Tensor, ws: list[torch.Tensor], tiled: bool, kind: str, gelu: 
     if residual is not None:  # before any launch: the kernel reads it through a raw pointer
         _check_residual(residual, x.device, (*x.shape[:-1], int(ws[0].size(0))))
     m = x.numel() // k
+    if not gelu and k == 2048 and 1 <= m <= SMALL_M_MAX_ROWS and x.is_cuda:
+        return _run_small(x, ws, k, m, tiled, kind, norm, residual)
     if k == 16384 and m >= E3M2_MIN_ROWS_K16384 and len(ws) == 1 and norm is None and not tiled:
         form = e3m2_form(ws[0], k)
         if form is not None and form.device == x.device:
             return _run_e3m2_rows(x, form, k, m, residual)
-    if not gelu and k == 2048 and 1 <= m <= SMALL_M_MAX_ROWS and x.is_cuda:
-        return _run_small(x, ws, k, m, tiled, kind, norm, residual)
     # the reference quantizes before checking the weights
     q, sa = quantize(x, warm) if norm is None else rms_norm_quantize(x, *norm, warm=warm)
     conv = []
