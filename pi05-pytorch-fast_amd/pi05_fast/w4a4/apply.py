@@ -90,9 +90,9 @@ def load_time_weight(
             register_int4_twin(w_e3m2, w_mfma, in_features)
             return w_e3m2, False
         # The down projection (K = 16384) keeps the INT4 form and registers its E3M2 form, on
-        # which calls of thousands of rows run.
+        # which calls of thousands of rows run (register_e3m2_form takes no inference tensors).
         if (os.environ.get("PI05_W4A4_E3M2", "1") != "0" and name.endswith(".mlp.down_proj")
-                and in_features == 16384 and out_features % 32 == 0):
+                and in_features == 16384 and out_features % 32 == 0 and not w_mfma.is_inference()):
             from pi05_fast.w4a4.extension import register_e3m2_form
 
             register_e3m2_form(w_mfma, repack_weight_e3m2(w_mfma, k=in_features, tiled=False), in_features)

@@ -519,11 +519,15 @@ _E3M2_FORMS: dict[int, tuple] = {}
 
 
 def register_e3m2_form(w_int4: torch.Tensor, w_e3m2: torch.Tensor, k: int) -> None:
-    """Record w_e3m2 as the E3M2 form of the MFMA-layout weight w_int4."""
+    """Record w_e3m2 as the E3M2 form of the MFMA-layout weight w_int4.  A weight made under
+    ``torch.inference_mode()`` has no version counter that would show a write in place: nothing
+    is recorded for it, and its calls stay on the INT4 kernels."""
     if not (is_e3m2_layout(w_e3m2, k) and is_mfma_layout(w_int4, k)):
         raise RuntimeError("register_e3m2_form takes an MFMA-layout weight and its E3M2-layout form")
     if int(w_e3m2.size(0)) != int(w_int4.size(0)):
         raise RuntimeError("the two forms of a weight must have the same N")
+    if w_int4.is_inference():
+        return
     key = id(w_int4)
     _E3M2_FORMS[key] = (weakref.ref(w_int4, lambda _r, key=key: _E3M2_FORMS.pop(key, None)), w_int4._version,
                         w_int4.data_ptr(), k, w_e3m2)

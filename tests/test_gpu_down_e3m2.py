@@ -104,6 +104,21 @@ def test_rule(ext, cuda, monkeypatch):
     assert not ext.int4_gemm(x, w4).any() and len(calls) == 5
 
 
+def test_weight_loaded_under_inference_mode(ext, cuda, monkeypatch):
+    """No E3M2 form is kept for it, and its calls run on the INT4 weight."""
+    from pi05_fast.w4a4.apply import load_time_weight
+
+    monkeypatch.setattr(ext, "E3M2_MIN_ROWS_K16384", 64)
+    gen = inp.generator(8400)
+    packed = inp.random_packed(gen, 64, K)
+    x = inp.geglu_activations(gen, 100, K).to(cuda)
+    want = ext.int4_gemm(x, packed.to(cuda))
+    with torch.inference_mode():
+        w, shuffled = load_time_weight(packed, "layers.0.mlp.down_proj", K, 64, torch.device(cuda))
+        assert not shuffled and ext.e3m2_form(w, K) is None
+        assert _same(ext.int4_gemm(x, w), want)
+
+
 def test_entry_refusals(ext, cuda):
     lib = ext.load_int4_gemm()
     b = torch.zeros(1 << 20, dtype=torch.uint8, device=cuda).data_ptr()

@@ -878,3 +878,32 @@ def test_int4_twin_registry():
     del w6
     gc.collect()
     assert key not in ext._INT4_TWINS
+
+
+def test_e3m2_form_registry():
+    """register_e3m2_form / e3m2_form on CPU tensors of the two layouts' shapes; weights made
+    under inference mode (no version counter) are taken and keep their INT4 form alone."""
+    from pi05_fast.w4a4 import extension as ext
+
+    k = 16384
+
+    def pair():
+        return (torch.zeros(64, k // 8 + 16, dtype=torch.int32), torch.zeros(64, 3 * k // 16 + 16, dtype=torch.int32))
+
+    w4, w6 = pair()
+    assert ext.e3m2_form(w4, k) is None
+    ext.register_e3m2_form(w4, w6, k)
+    assert ext.e3m2_form(w4, k) is w6 and ext.e3m2_form(w4, 2048) is None
+    w4.zero_()  # written in place: the form no longer stands for it
+    assert ext.e3m2_form(w4, k) is None
+    with pytest.raises(RuntimeError):
+        ext.register_e3m2_form(w6, w4, k)
+    with torch.inference_mode():
+        i4, i6 = pair()
+        ext.register_e3m2_form(i4, i6, k)
+        assert ext.e3m2_form(i4, k) is None
+    assert ext.e3m2_form(i4, k) is None
+    w4, w6 = pair()
+    ext.register_e3m2_form(w4, w6, k)
+    ext.clear_weight_caches()
+    assert ext.e3m2_form(w4, k) is None
