@@ -77,8 +77,8 @@ int pi05w4a4_quantize(const void* x_fp16, int64_t m, int32_t k, int32_t* q, floa
                       void* stream);
 
 /*
- * pi05w4a4_quantize plus cache warming: at K = 16384 (one 68 KB workgroup per row, two per
- * CU) the workgroup slots that the last round of rows leaves idle read warm_n <= 4 further
+ * pi05w4a4_quantize plus cache warming: at K = 16384 (a workgroup per row, two per CU,
+ * three beyond four rows per CU) the workgroup slots that the last round of rows leaves idle read warm_n <= 4 further
  * device buffers (16-byte aligned, sizes multiples of 16 bytes) and discard the data, so
  * that the kernels after it find them in the Infinity Cache; other K ignore the buffers.
  * No counterpart in the reference: the fused decoder layer passes the down-proj weights
@@ -428,7 +428,8 @@ int pi05w4a4_prefix_attention_warm(const void* q, int64_t ld_q, const void* kv_m
  * pi05w4a4_gemm_e3m2: gelu_up = 0: pi05w4a4_gemm_multi of 1..3 w6 weights (n[g] columns
  *   into y[g]); gelu_up = 1: pi05w4a4_gemm_gelu_up (ngroups = 2: gate, up with
  *   n[0] == n[1]; y[0] = fp16(gelu_tanh(gate) * up)).  One launch, no workspace.
- * pi05w4a4_quantize_e3m2_k16384: pi05w4a4_quantize at K = 16384 with the codes written as q6.
+ * pi05w4a4_quantize_e3m2_k16384: pi05w4a4_quantize at K = 16384 with the codes written as q6;
+ *   pi05w4a4_quantize_e3m2_k16384_warm: the same plus pi05w4a4_quantize_warm's cache warming.
  * pi05w4a4_gemm_e3m2_rows: pi05w4a4_gemm, or with residual_fp16 (may be null)
  *   pi05w4a4_gemm_residual, on E3M2 operands with tiles for thousands of rows.
  */
@@ -445,6 +446,9 @@ int pi05w4a4_gemm_e3m2(const void* q6, const float* sa, int64_t m, int32_t k, in
                        const int32_t* const* w6, const int32_t* n, void* const* y_fp16, int32_t gelu_up,
                        void* stream);
 int pi05w4a4_quantize_e3m2_k16384(const void* x_fp16, int64_t m, void* q6, float* sa, void* stream);
+int pi05w4a4_quantize_e3m2_k16384_warm(const void* x_fp16, int64_t m, void* q6, float* sa,
+                                       const void* const* warm_ptrs, const size_t* warm_bytes, int32_t warm_n,
+                                       void* stream);
 int pi05w4a4_gemm_e3m2_rows(const void* q6, const float* sa, int64_t m, int32_t k, const int32_t* w6, int32_t n,
                             const void* residual_fp16, void* y_fp16, void* stream);
 

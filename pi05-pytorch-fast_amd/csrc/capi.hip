@@ -716,7 +716,9 @@ int pi05w4a4_gemm_e3m2(const void* q6, const float* sa, int64_t m, int32_t k, in
   return hip_status(w4a4::launch_gemm_e3m2(p, tile_cfg, static_cast<hipStream_t>(stream)), "E3M2 gemm launch");
 }
 
-int pi05w4a4_quantize_e3m2_k16384(const void* x_fp16, int64_t m, void* q6, float* sa, void* stream) {
+namespace {
+int quantize_e3m2_k16384_call(const void* x_fp16, int64_t m, void* q6, float* sa, const w4a4::CacheWarmParams* warm,
+                              void* stream) {
   if (m < 0) return fail(PI05W4A4_EINVAL, "M must be >= 0, got %lld", (long long)m);
   if (m == 0) return ok();
   if (!x_fp16 || !q6 || !sa) return fail(PI05W4A4_EINVAL, "null pointer argument");
@@ -725,8 +727,22 @@ int pi05w4a4_quantize_e3m2_k16384(const void* x_fp16, int64_t m, void* q6, float
   if (m > 0x7fffffffLL) return fail(PI05W4A4_EINVAL, "M too large");
   return hip_status(w4a4::launch_quantize_e3m2(x_fp16, nullptr, 0.0f, 0, m, 16384, q6, sa,
                                                static_cast<float>(1.0 / std::sqrt(16384.0)),
-                                               static_cast<hipStream_t>(stream), nullptr),
+                                               static_cast<hipStream_t>(stream), warm),
                     "E3M2 quantize launch");
+}
+}  // namespace
+
+int pi05w4a4_quantize_e3m2_k16384(const void* x_fp16, int64_t m, void* q6, float* sa, void* stream) {
+  return quantize_e3m2_k16384_call(x_fp16, m, q6, sa, nullptr, stream);
+}
+
+int pi05w4a4_quantize_e3m2_k16384_warm(const void* x_fp16, int64_t m, void* q6, float* sa,
+                                       const void* const* warm_ptrs, const size_t* warm_bytes, int32_t warm_n,
+                                       void* stream) {
+  w4a4::CacheWarmParams warm;
+  const int rc = collect_warm(warm_ptrs, warm_bytes, warm_n, &warm);
+  if (rc) return rc;
+  return quantize_e3m2_k16384_call(x_fp16, m, q6, sa, &warm, stream);
 }
 
 int pi05w4a4_gemm_e3m2_rows(const void* q6, const float* sa, int64_t m, int32_t k, const int32_t* w6, int32_t n,

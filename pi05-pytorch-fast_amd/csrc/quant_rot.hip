@@ -496,9 +496,12 @@ hipError_t launch_quantize_e3m2(const void* x, const void* nw, float eps, int un
                                 int32_t k, void* q6, float* sa, float inv_sqrt_k, hipStream_t stream,
                                 const CacheWarmParams* warm) {
   if (m <= 0) return hipSuccess;
-  if (k == 16384 && nw == nullptr) {
-    fwht_quant_kernel<14, 8, 1, false, true, true><<<dim3(static_cast<unsigned>(m)), 256, 0, stream>>>(
-        static_cast<const _Float16*>(x), m, static_cast<int32_t*>(q6), sa, nullptr, inv_sqrt_k);
+  if (k == 16384 && nw == nullptr) {  // half rows, three workgroups per CU; warming as in launch_quantize
+    const int64_t slots = 3 * static_cast<int64_t>(device_cu_count());
+    const int64_t extra = (warm != nullptr && warm->nbuf > 0 && m % slots != 0) ? slots - m % slots : 0;
+    fwht_quant_kernel<14, 8, 1, false, true, true><<<dim3(static_cast<unsigned>(m + extra)), 256, 0, stream>>>(
+        static_cast<const _Float16*>(x), m, static_cast<int32_t*>(q6), sa, nullptr, inv_sqrt_k, nullptr, 0.0f, 0,
+        extra > 0 ? *warm : CacheWarmParams{});
     return hipGetLastError();
   }
   if (k != 2048) return hipErrorInvalidValue;

@@ -240,7 +240,7 @@ hipError_t launch_repack(const int32_t* src, int32_t layout, int32_t n, int32_t 
 // INT4 MFMA-layout weight (N % 32 == 0, K % 128 == 0) -> the E3M2 pair layout w6.
 hipError_t launch_repack_e3m2(const int32_t* w_mfma, int32_t n, int32_t k, int32_t* dst, hipStream_t stream);
 // K = 2048 activation quant (optionally with the fused RMSNorm, nw != null) or K = 16384 quant
-// (no norm, no warming) writing E3M2 fragments (q6) instead of INT4 codes.
+// (no norm) writing E3M2 fragments (q6) instead of INT4 codes.
 hipError_t launch_quantize_e3m2(const void* x, const void* nw, float eps, int unit_offset, int64_t m,
                                 int32_t k, void* q6, float* sa, float inv_sqrt_k, hipStream_t stream,
                                 const CacheWarmParams* warm = nullptr);

@@ -143,6 +143,8 @@ def load_int4_gemm():
                            vp]),
         "pi05w4a4_gemm_e3m2": (ctypes.c_int, [vp, vp, i64, i32, i32, vp, vp, vp, i32, vp]),
         "pi05w4a4_quantize_e3m2_k16384": (ctypes.c_int, [vp, i64, vp, vp, vp]),
+        "pi05w4a4_quantize_e3m2_k16384_warm": (
+            ctypes.c_int, [vp, i64, vp, vp, ctypes.POINTER(vp), ctypes.POINTER(sz), i32, vp]),
         "pi05w4a4_gemm_e3m2_rows": (ctypes.c_int, [vp, vp, i64, i32, vp, i32, vp, vp, vp]),
     }
     for name, (res, args) in sig.items():
@@ -858,7 +860,9 @@ def _run(x: torch.Tensor, ws: list[torch.Tensor], tiled: bool, kind: str, gelu: 
     if k == 16384 and m >= E3M2_MIN_ROWS_K16384 and len(ws) == 1 and norm is None and not tiled:
         form = e3m2_form(ws[0], k)
         if form is not None and form.device == x.device:
-            return _run_e3m2_rows(x, form, k, m, residual)
+            if warm:  # a list that names the weight means what the call reads
+                warm = [form if t is ws[0] else t for t in warm]
+            return _run_e3m2_rows(x, form, k, m, residual, warm)
     # the reference quantizes before checking the weights
     q, sa = quantize(x, warm) if norm is None else rms_norm_quantize(x, *norm, warm=warm)
     conv = []
@@ -935,7 +939,7 @@ def _run_e3m2(x, ws, k, n_e3m2, kind, gelu, norm, residual, warm=None):
         return _gemm_e3m2_from_q(q6, sa, k, ws, tuple(x.shape[:-1]), dev, gelu=gelu)
 
 
-def _run_e3m2_rows(x, w6, k, m, residual):
+def _run_e3m2_rows(x, w6, k, m, residual, warm=None):
     """_run for one K = 16384 weight at thousands of rows, on its E3M2 form w6."""
     x2 = x if x.is_contiguous() else x.contiguous()
     if x2.data_ptr() % 16:
@@ -951,8 +955,13 @@ def _run_e3m2_rows(x, w6, k, m, residual):
     out = torch.empty((m, n), dtype=torch.float16, device=dev)
     with _on_device(dev):
         st = _stream(dev)
-        _check(lib.pi05w4a4_quantize_e3m2_k16384(x2.data_ptr(), m, q6.data_ptr(), sa.data_ptr(), st),
-               "pi05w4a4_quantize_e3m2_k16384")
+        wa = _warm_args(warm, "quantize") if warm else None
+        if wa is None:
+            _check(lib.pi05w4a4_quantize_e3m2_k16384(x2.data_ptr(), m, q6.data_ptr(), sa.data_ptr(), st),
+                   "pi05w4a4_quantize_e3m2_k16384")
+        else:
+            _check(lib.pi05w4a4_quantize_e3m2_k16384_warm(x2.data_ptr(), m, q6.data_ptr(), sa.data_ptr(), *wa, st),
+                   "pi05w4a4_quantize_e3m2_k16384_warm")
         _check(lib.pi05w4a4_gemm_e3m2_rows(q6.data_ptr(), sa.data_ptr(), m, k, w6.data_ptr(), n, _ptr(res),
                                            out.data_ptr(), st), "pi05w4a4_gemm_e3m2_rows")
     return [out.view(*x.shape[:-1], n)]

@@ -104,6 +104,27 @@ def test_rule(ext, cuda, monkeypatch):
     assert not ext.int4_gemm(x, w4).any() and len(calls) == 5
 
 
+@pytest.mark.parametrize("m", [256, 768, 1000])
+def test_warming(ext, cuda, monkeypatch, m):
+    """Buffers to warm change nothing in the outputs, the weight in them stands for the form that
+    the call reads, and what the quantizer refuses stays refused."""
+    monkeypatch.setattr(ext, "E3M2_MIN_ROWS_K16384", 256)
+    gen = inp.generator(8500 + m)
+    w4, w6 = _weight(ext, gen, 64, cuda)
+    x, r = inp.geglu_activations(gen, m, K).to(cuda), torch.randn(m, 64, generator=gen).half().to(cuda)
+    want = ext.int4_gemm_residual(x, w4, r)
+    ext.register_e3m2_form(w4, w6, K)
+    big = torch.ones(1 << 20, dtype=torch.uint8, device=cuda)
+    seen = []
+    real = ext._warm_args
+    monkeypatch.setattr(ext, "_warm_args", lambda warm, who: seen.append(list(warm)) or real(warm, who))
+    assert _same(ext.int4_gemm_residual(x, w4, r, warm=[w4, big]), want)
+    assert len(seen) == 1 and seen[0][0] is w6 and seen[0][1].data_ptr() == big.data_ptr()
+    for bad in ([big.cpu()], [big[::2]], [big] * 5):
+        with pytest.raises(RuntimeError):
+            ext.int4_gemm_residual(x, w4, r, warm=bad)
+
+
 def test_weight_loaded_under_inference_mode(ext, cuda, monkeypatch):
     """No E3M2 form is kept for it, and its calls run on the INT4 weight."""
     from pi05_fast.w4a4.apply import load_time_weight

@@ -427,6 +427,16 @@ def test_attention_abi_validation_without_gpu(lib):
     assert qwarm([p], [1024], k=100) == 1 and "multiple of 64" in _err(lib)
     assert qwarm([p], [1024], x=vp(0)) == 1 and "null" in _err(lib)
 
+    # and its E3M2 form
+    def ewarm(ptrs, sizes, x=p):
+        arr = (vp * max(len(ptrs), 1))(*ptrs)
+        sz = (ctypes.c_size_t * max(len(sizes), 1))(*sizes)
+        return lib.pi05w4a4_quantize_e3m2_k16384_warm(x, 776, p, p, arr, sz, len(ptrs), vp(0))
+
+    assert ewarm([p] * 5, [16] * 5) == 1 and "0..4 buffers" in _err(lib)
+    assert ewarm([vp(264)], [1024]) == 1 and "16-byte aligned" in _err(lib)
+    assert ewarm([p], [1024], x=vp(0)) == 1 and "null" in _err(lib)
+
 
 # ----------------------------------------------------------------------------- op surface
 def test_custom_ops_registered_with_fakes():
