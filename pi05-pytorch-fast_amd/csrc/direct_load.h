@@ -29,5 +29,12 @@ __device__ __forceinline__ void wait_vm() {
 // This wave's LDS operations are done, and every wave of the workgroup has come here.
 __device__ __forceinline__ void lds_done_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// A copy that the compiler cannot know to equal v: what is computed from it inside a loop stays
+// there, and takes no register across the loop's other parts.
+__device__ __forceinline__ int opaque_copy(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
 }  // namespace
 }  // namespace w4a4

@@ -7,7 +7,12 @@
 // register ring.  The column pairs of a block are multiplied one after the other, so that a
 // pair's registers are free half a step before the block ends and take the pair of the block
 // after the next: the lead of a three-block ring in the registers of two (a three-block ring
-// spills).  The workgroups walk the tiles, and the loads run on into the next tile's first
+// spills).  Two workgroups per CU leave a wave 256 registers, of which the 112-row plain tile
+// takes all (accumulators 112, column pairs 48, row fragments 42): per-lane offsets of the next
+// tile's rows and of the epilogue are made where they are used (opaque_copy), and the residual's
+// are 32-bit ones from a uniform base.  Kept over the k loop they spilled 180 bytes, and each
+// reload waited for every load under way: down projection with residual at 6208 rows 219.9 us with
+// its quantizer, 206.4 now.  The workgroups walk the tiles, and the loads run on into the next tile's first
 // blocks, so that the loads' latency is paid once per workgroup and not once per tile.
 // The direct loads are inline asm (they write LDS only, no register): the compiler orders
 // every LDS read behind all earlier direct-to-LDS loads that it knows of, which would empty
@@ -67,8 +72,6 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
 
   const int nkb = kblocks128(p.k);
   const int64_t M = p.m;
-  const int lrow = lane & 15;
-  const int lcol = (lane >> 4) * 4;
 
   // ---- tiles of this workgroup.  XCD x = b % 8 owns a contiguous run of the tiles in an
   // order that walks the m-tiles of one m-group under each n-tile, n-tiles outside, m-groups
@@ -124,14 +127,15 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
   const uint32_t frag_stride = static_cast<uint32_t>(nkb) * kE3m2FragBytes;  // one row block's k blocks
   auto a_start = [&](const Tile& c, const char*& base, uint32_t (&off)[T::kPerWave]) {
     const int mb0 = c.mt * MI;
+    const int l = opaque_copy(lane);  // made at the tile's start, not kept
     base = reinterpret_cast<const char*>(p.q) + static_cast<int64_t>(mb0) * frag_stride;
 #pragma unroll
     for (int j = 0; j < T::kPerWave; ++j) {
       const int pc = min(wave + T::kWaves * j, T::kChunks - 1);
       const bool lo = pc < MI;
-      const int f = lo ? pc : min(2 * (pc - MI) + (lane >> 5), MI - 1);
+      const int f = lo ? pc : min(2 * (pc - MI) + (l >> 5), MI - 1);
       const int rel = min(mb0 + f, p.mblocks - 1) - mb0;
-      off[j] = static_cast<uint32_t>(rel) * frag_stride + (lo ? lane * 16 : 1024 + (lane & 31) * 16);
+      off[j] = static_cast<uint32_t>(rel) * frag_stride + (lo ? l * 16 : 1024 + (l & 31) * 16);
     }
   };
   const char* abase;
@@ -189,8 +193,7 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
   // the pair's registers pair 1 of block kb + 2; the wave's loads of A stage kb + 3 are spread
   // among them.  Blocks and stages past the tile's last are the next tile's.
   bool more = false;  // there is a next tile
-  const char* abase_next;
-  uint32_t voff_next[T::kPerWave];
+  Tile nxt = tile_at(t_next);
   auto step = [&](int kb, v12i (&b)[2]) {
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi)
@@ -220,11 +223,7 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
 #pragma unroll
         for (int j = 0; j < T::kPerWave; ++j) issue_a(j, wr);
         abase += kE3m2FragBytes;
-        if (kb + 4 == nkb && more) {
-          abase = abase_next;
-#pragma unroll
-          for (int j = 0; j < T::kPerWave; ++j) voff[j] = voff_next[j];
-        }
+        if (kb + 4 == nkb && more) a_start(nxt, abase, voff);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -276,8 +275,7 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
   for (;;) {
     t_next += t_stride;
     more = t_next < t_end;
-    const Tile nxt = tile_at(more ? t_next : t_next - t_stride);
-    a_start(nxt, abase_next, voff_next);
+    nxt = tile_at(more ? t_next : t_next - t_stride);
 #pragma unroll
     for (int qd = 0; qd < 2; ++qd) bp_next[qd] = b_start(nxt, qd);
 #pragma unroll
@@ -296,6 +294,10 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
     }
     const int64_t m0 = static_cast<int64_t>(cur.mt) * (16 * MI);
     const int wcol = cur.wcol, N = cur.n;
+    // The epilogue's per-lane offsets are made from a copy, so that they are not kept over the k loop.
+    const int elane = opaque_copy(lane);
+    const int lrow = elane & 15;
+    const int lcol = (elane >> 4) * 4;
     // Epilogue scales: the lane's row of every row fragment and its four columns of every
     // column fragment (clamped: rows and columns past the matrix are never stored).
     float sv[MI];
@@ -319,18 +321,22 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
   _Float16* const stage = reinterpret_cast<_Float16*>(lds + T::kOut) + wave * (16 * LSR);
   const int8_t* const fix = reinterpret_cast<const int8_t*>(lds + T::kFix);
   char* const yw = reinterpret_cast<char*>(cur.y + m0 * N + wcol);
-  const uint32_t loff = static_cast<uint32_t>((lane / LPR) * N + (lane % LPR) * 8) * 2u;
+  const uint32_t loff = static_cast<uint32_t>((elane / LPR) * N + (elane % LPR) * 8) * 2u;
   // Residual: the 16-byte pieces that this wave's store loop adds, two row blocks ahead
   // (addresses clamped into the matrix; pieces outside it are never stored).
   const bool has_res = !GELU && p.res != nullptr;
   uint4 resv[GELU ? 1 : 3][16 / RPI];
+  const int rmax = static_cast<int>(min(M - 1 - m0, static_cast<int64_t>(16 * MI - 1)));  // last row of the tile
+  const uint32_t rcol = static_cast<uint32_t>(min(wcol + (elane % LPR) * 8, N - 8)) * 2u;
   auto load_res = [&](int mi) {
     if constexpr (!GELU) {
       if (mi < MI && has_res) {
-        const _Float16* const rcol = p.res + min(wcol + (lane % LPR) * 8, N - 8);
+        const char* const rb = reinterpret_cast<const char*>(p.res + m0 * N);
 #pragma unroll
-        for (int j = 0; j < 16 / RPI; ++j)
-          resv[mi % 3][j] = *reinterpret_cast<const uint4*>(rcol + min(m0 + mi * 16 + j * RPI + lane / LPR, M - 1) * N);
+        for (int j = 0; j < 16 / RPI; ++j) {
+          const uint32_t r = static_cast<uint32_t>(min(mi * 16 + j * RPI + elane / LPR, rmax));
+          resv[mi % 3][j] = *reinterpret_cast<const uint4*>(rb + (r * static_cast<uint32_t>(2 * N) + rcol));
+        }
       }
     }
   };
@@ -368,8 +374,8 @@ __device__ __forceinline__ void e3m2_tile(const GemmParams& p, char* lds, const 
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int j = 0; j < 16 / RPI; ++j) {
-      const int rr = j * RPI + lane / LPR;
-      const int tcol = (lane % LPR) * 8;
+      const int rr = j * RPI + elane / LPR;
+      const int tcol = (elane % LPR) * 8;
       const int trow = mi * 16 + rr;
       uint4 v = *reinterpret_cast<const uint4*>(stage + rr * LSR + tcol);
       char* const yrow = yw + static_cast<int64_t>(mi * 16 + j * RPI) * N * 2;  // uniform; + loff per lane

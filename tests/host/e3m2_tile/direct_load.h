@@ -37,6 +37,7 @@ void wait_vm() {
   }
 }
 inline void lds_done_barrier() { barrier(); }
+inline int opaque_copy(int v) { return v; }
 
 }  // namespace
 }  // namespace w4a4
