@@ -509,15 +509,48 @@ def int4_twin(w: torch.Tensor, k: int) -> torch.Tensor | None:
 
 
 # E3M2 forms of INT4 MFMA-layout K = 16384 weights (the down projection), registered by the
-# loader: calls of at least E3M2_MIN_ROWS_K16384 rows run on them.  The INT4 kernel's 112 x 64
-# tiles of eight K-split waves take a CU each: 1792 rows of N = 2048 are two full rounds of 256
-# CUs, and every further 896 rows a round more, while the E3M2 tile's 112 x 256 tiles pay one
-# workgroup time up to 3584 rows.  Measured (activation quant + GEMM + residual, us, INT4 /
-# E3M2): 1500 rows 83 / 92, 1792 86 / 96, 1793 98 / 96, 2128 107 / 101, 2688 134 / 107, 3584
-# 189 / 121, 4480 235 / 170, 6208 243 / 222.  An entry lives as long as its INT4 weight and is
-# ignored once that weight is modified in place, like a twin's.
-E3M2_MIN_ROWS_K16384 = 1793
+# loader: the calls of e3m2_form_pays run on them.  An entry lives as long as its INT4 weight and
+# is ignored once that weight is modified in place, like a twin's.
 _E3M2_FORMS: dict[int, tuple] = {}
+# A row count in place of e3m2_form_pays (None: the rule decides).
+E3M2_MIN_ROWS_K16384: int | None = None
+_CU_COUNT: dict[int, int] = {}
+
+
+def e3m2_form_pays(m: int, n: int, cus: int) -> bool:
+    """Whether a K = 16384 call of m rows and n columns is faster on the weight's E3M2 form.
+
+    The INT4 kernel's 112 x 64 tiles of eight K-split waves take a CU each, so their rounds of CUs
+    count; the E3M2 tile's 112 x 256 tiles pay one workgroup time (of about 2.4 INT4 rounds) up to
+    a tile per CU.  So the form is taken from the round on that makes the INT4 tiles the longer
+    way; at many rows, where the INT4 tiles' repeated reads of the rows count too, within the last
+    quarter of the second round.  Calls of up to seven rows per CU stay on INT4 (from N = 2560 on
+    the form would be faster for some of them, 4096 columns at 1456 rows 107 / 80).
+    Measured (256 CUs; quant + GEMM + residual, us, INT4 / E3M2):
+      N = 64: 1793 rows 46 / 82, 6208 95 / 129; N = 256: 7168 122 / 145, 14448 250 / 247;
+      N = 512: 3584 81 / 100, 6208 136 / 132, 7168 156 / 157, 7280 173 / 155;
+      N = 1024: 1793 67 / 82, 2688 88 / 91, 3584 117 / 100; N = 1536: 2352 89 / 90, 2464 106 / 89;
+      N = 2048: 1792 74 / 82, 1793 90 / 82, 2688 130 / 94, 3584 180 / 107, 4480 224 / 151, 6208
+      218 / 197; N = 4096: 1793 138 / 125, 6208 352 / 322."""
+    mt = -(-m // 112)
+    tiles4 = mt * -(-n // 64)
+    rounds4, rounds6 = -(-tiles4 // cus), -(-(mt * -(-n // 256)) // cus)
+    if m <= 7 * cus:
+        return False
+    return 5 * rounds4 > 12 * rounds6 or (n >= 512 and m > 12 * cus and 4 * tiles4 >= 7 * cus)
+
+
+def _form_for_rows(w: torch.Tensor, k: int, m: int, device: torch.device) -> torch.Tensor | None:
+    """The E3M2 form of w (on ``device``) for a call of m rows, or None: the call stays on w."""
+    cus = _CU_COUNT.get(device.index)
+    if cus is None:
+        cus = _CU_COUNT[device.index] = torch.cuda.get_device_properties(device).multi_processor_count
+    if m < (7 * cus if E3M2_MIN_ROWS_K16384 is None else E3M2_MIN_ROWS_K16384):  # most calls: no look-up
+        return None
+    form = e3m2_form(w, k)
+    if form is None or form.device != device:
+        return None
+    return form if E3M2_MIN_ROWS_K16384 is not None or e3m2_form_pays(m, int(form.size(0)), cus) else None
 
 
 def register_e3m2_form(w_int4: torch.Tensor, w_e3m2: torch.Tensor, k: int) -> None:
@@ -857,9 +890,9 @@ def _run(x: torch.Tensor, ws: list[torch.Tensor], tiled: bool, kind: str, gelu: 
     m = x.numel() // k
     if not gelu and k == 2048 and 1 <= m <= SMALL_M_MAX_ROWS and x.is_cuda:
         return _run_small(x, ws, k, m, tiled, kind, norm, residual)
-    if k == 16384 and m >= E3M2_MIN_ROWS_K16384 and len(ws) == 1 and norm is None and not tiled:
-        form = e3m2_form(ws[0], k)
-        if form is not None and form.device == x.device:
+    if k == 16384 and len(ws) == 1 and norm is None and not tiled:
+        form = _form_for_rows(ws[0], k, m, x.device)
+        if form is not None:
             if warm:  # a list that names the weight means what the call reads
                 warm = [form if t is ws[0] else t for t in warm]
             return _run_e3m2_rows(x, form, k, m, residual, warm)

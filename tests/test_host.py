@@ -917,3 +917,20 @@ def test_e3m2_form_registry():
     ext.register_e3m2_form(w4, w6, k)
     ext.clear_weight_caches()
     assert ext.e3m2_form(w4, k) is None
+
+
+def test_e3m2_form_rule():
+    """Which K = 16384 calls run on a weight's E3M2 form: sides of the rule at several widths, the
+    same line per CU on a device of half the CUs, and one side only as the rows grow."""
+    from pi05_fast.w4a4.extension import e3m2_form_pays as pays
+
+    assert not pays(1792, 2048, 256) and pays(1793, 2048, 256) and pays(6208, 2048, 256)
+    assert not pays(896, 2048, 128) and pays(897, 2048, 128)
+    for n in (32, 64, 128):  # narrower than an E3M2 tile: INT4 up to any row count
+        assert not any(pays(m, n, 256) for m in range(1, 40000, 111))
+    assert not pays(7168, 256, 256) and not pays(3584, 512, 256) and pays(6208, 512, 256)
+    assert not pays(1793, 1024, 256) and pays(3584, 1024, 256) and not pays(2352, 1536, 256) and pays(2464, 1536, 256)
+    assert not pays(1792, 8192, 256) and pays(1793, 8192, 256)
+    for n in (512, 1024, 2048, 4096):
+        side = [pays(m, n, 256) for m in range(1, 20000, 16)]
+        assert side == sorted(side)
