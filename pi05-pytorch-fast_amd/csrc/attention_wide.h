@@ -13,10 +13,9 @@
 //                 fp32 row sum, O / sum at the end.  m moves (and O and the sum are rescaled)
 //                 only when a score exceeds it by more than 8 in log2 units, so that p stays
 //                 below 2^8 and the check needs no exchange between lanes.
-// The direct loads are inline asm (they write LDS only, no register), since the compiler
-// would drain them before every LDS read; the full wait and the barrier at the top of a step
-// order them.  The mask of the next step is loaded after this one's was used and handed over
-// behind that same wait.
+// The direct loads (direct_load.h) stay in flight over the LDS reads of a step; the full wait
+// and the barrier at the top of a step order them.  The mask of the next step is loaded after
+// this one's was used and handed over behind that same wait.
 //
 // What bounds it (776 tokens x 8, 392 workgroups, one or two per CU): a step of a workgroup
 // that has its CU for itself takes ~2300 cycles, 1024 of them MFMAs, ~600 the softmax's vector
@@ -33,6 +32,7 @@
 // (s_setprio) during the MFMAs 71.5 / 64.8, during the softmax 67.7 / 64.9.
 #pragma once
 
+#include "direct_load.h"
 #include "quant_row.h"
 
 namespace w4a4 {
@@ -48,13 +48,6 @@ constexpr int kWideStage = 32 * 1024;  // K (16 pieces of 1 KB), then V^T (16)
 constexpr size_t kWideLds = 2 * kWideStage;
 constexpr size_t kWideLdsQuant = sizeof(_Float16) * (kWideRows / 8) * kOld;  // the staged output tokens
 static_assert(kWideLdsQuant >= kWideLds, "the staged tokens reuse the stages");
-
-// One 1 KB piece from global memory (uniform base + per-lane byte offset) to LDS address
-// `dst` (lane L writes bytes 16 L ..).  No other instruction of the kernel uses m0.
-__device__ __forceinline__ void attn_load_lds_1k(const char* base, uint32_t voff, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               ::"v"(voff), "s"(base), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory");
-}
 
 // Packed fp16 max as one instruction (the compiler's form quiets its operands first).
 __device__ __forceinline__ uint32_t pk_max(uint32_t a, uint32_t b) {
@@ -99,9 +92,9 @@ __global__ __launch_bounds__(kWideThreads, 2) void prefix_attention_wide_kernel(
   auto load_piece = [&](int u, int u1, int j) {  // j = 0..3: K, 4..7: V^T
     const uint32_t st = lds0 + (u & 1) * kWideStage + 4 * w * 1024;
     if (j < 4)
-      attn_load_lds_1k(kt + static_cast<int64_t>(u1) * 16384 + (4 * (w & 1) + j) * 1024, koff, st + j * 1024);
+      load_lds_1k(kt + static_cast<int64_t>(u1) * 16384 + (4 * (w & 1) + j) * 1024, koff, st + j * 1024);
     else
-      attn_load_lds_1k(vt + (static_cast<int64_t>(4 * w + j - 4) * nst + u1) * 1024, voff, st + 16384 + (j - 4) * 1024);
+      load_lds_1k(vt + (static_cast<int64_t>(4 * w + j - 4) * nst + u1) * 1024, voff, st + 16384 + (j - 4) * 1024);
   };
 
   // Mask chunks of a step: row 16 qb + L % 16, keys 8 (L / 16) + 0..7, in 8-byte halves

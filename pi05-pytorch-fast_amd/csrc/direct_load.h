@@ -11,10 +11,10 @@ namespace w4a4 {
 namespace {
 
 // One 1 KB piece from global memory (uniform base + per-lane byte offset) to LDS address
-// `dst` (lane L writes bytes 16 L ..).  No other instruction of the kernel uses m0.
+// `dst` (lane L writes bytes 16 L ..).
 __device__ __forceinline__ void load_lds_1k(const char* base, uint32_t voff, uint32_t dst) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               ::"v"(voff), "s"(base), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory");
+               ::"v"(voff), "s"(base), "s"(__builtin_amdgcn_readfirstlane(dst)) : "memory", "m0");
 }
 
 // An ordinary 16-byte load to registers, named because the wait counts include it.

@@ -14,11 +14,8 @@
 // reload waited for every load under way: down projection with residual at 6208 rows 219.9 us with
 // its quantizer, 206.4 now.  The workgroups walk the tiles, and the loads run on into the next tile's first
 // blocks, so that the loads' latency is paid once per workgroup and not once per tile.
-// The direct loads are inline asm (they write LDS only, no register): the compiler orders
-// every LDS read behind all earlier direct-to-LDS loads that it knows of, which would empty
-// the ring at every step.  The vmcnt waits and the barrier of a step are their ordering; the
-// compiler's own waits for the register loads do not count them, and so only wait for more.
-// No other instruction of the kernel uses m0.
+// The vmcnt waits and the barrier of a step order the direct loads (direct_load.h), whose lead over
+// the LDS reads is the ring's.
 //
 // What bounds it (gate/up + GELU at 6208 rows, times with parts of the kernel taken out of a
 // scratch copy): MFMAs, LDS reads and barriers alone 143 us (register operands alone 120: the

@@ -59,3 +59,10 @@ def test_no_register_spills(tmp_path):
     scratch = dict(re.findall(r"\.set (\S*gemm_w4a4_kernel\S*)\.private_seg_size, (\d+)", asm.read_text()))
     tiles = {n: int(v) for n, v in scratch.items() if re.search(r"ILi[4-7]ELi4ELi4ELi1ELb[01]ELi2ELi2ELb0ELb0ELb1E", n)}
     assert len(tiles) == 8 and not any(tiles.values()), tiles
+
+
+def test_direct_loads_declare_their_register():
+    """m0, which the direct loads' asm writes, is among what it clobbers, and one helper has it."""
+    writes = {f.name: f.read_text().count("s_mov_b32 m0") for f in CSRC.iterdir()}
+    assert {n: c for n, c in writes.items() if c} == {"direct_load.h": 1}
+    assert re.search(r's_mov_b32 m0[^;]*"m0"\)', (CSRC / "direct_load.h").read_text())
