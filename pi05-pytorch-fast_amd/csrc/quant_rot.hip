@@ -209,7 +209,7 @@ __global__ __launch_bounds__(ROWS << LOGT, HALF ? 3 : 1) void fwht_quant_kernel(
   __shared__ float red[ROWS * (T / 64 > 0 ? T / 64 : 1)];
   __shared__ int ired[T / 64];
 
-  const int sub = threadIdx.x >> LOGT;
+  const int sub = ROWS == 1 ? 0 : threadIdx.x >> LOGT;  // one row: its number is uniform
   const int t = threadIdx.x & (T - 1);
   const int64_t row = static_cast<int64_t>(xcd_row_group<ROWS>(blockIdx.x, static_cast<uint32_t>(m))) * ROWS + sub;
   if constexpr (T > 64) {
@@ -419,7 +419,8 @@ hipError_t launch_quantize(const void* x, int64_t m, int32_t k, int32_t* q, floa
   const dim3 grid(static_cast<unsigned>(m));
   switch (k) {
     case 16384: {
-      // Half-row transposes (36 KB of LDS, 131 VGPRs: three workgroups per CU) beyond four rows
+      // Half-row transposes (36 KB of LDS, 133 VGPRs, writing E3M2 168, which is the
+      // most that leaves room for three: three workgroups per CU) beyond four rows
       // per CU, whole rows (68 KB: two) up to there, where one row's own time counts.  Measured
       // (whole / half, us): 776 rows 14.8 / 16.0, 1024 16.1 / 17.5, 1552 26.0 / 24.0, 3104
       // 44.4 / 39.3, 6208 80.3 / 69.6.  Cache warming fills the slots that the last round of

@@ -44,21 +44,24 @@ def test_the_emulation_notices_a_count_that_is_too_large(tmp_path, loose):
             assert f"MI {mi} {form}, 16 k blocks" in run.stdout
 
 
-def test_no_register_spills(tmp_path):
-    """The tile's kernels keep everything in registers: a spilled value's reload waits for all the
-    loads that the rings hold in flight."""
+@pytest.mark.parametrize("unit,kernels,count", [
+    ("gemm.hip", r"gemm_w4a4_kernelILi[4-7]ELi4ELi4ELi1ELb[01]ELi2ELi2ELb0ELb0ELb1E", 8),
+    ("quant_rot.hip", r"fwht_quant_kernelILi14E", 3)])
+def test_no_register_spills(tmp_path, unit, kernels, count):
+    """The main tile's kernels keep everything in registers (a spilled value's reload waits for all
+    the loads that the rings hold in flight), and so do the K = 16384 quantizers."""
     spec = importlib.util.spec_from_file_location("_build_lib", CSRC.parent / "build_lib.py")
     build_lib = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(build_lib)
     cmds, _ = build_lib.compile_commands(["gfx950"], tmp_path)
-    cmd = next(c for c in cmds if c[c.index("-c") + 1].endswith("gemm.hip"))
-    asm = tmp_path / "gemm.s"
+    cmd = next(c for c in cmds if c[c.index("-c") + 1].endswith(unit))
+    asm = tmp_path / "unit.s"
     cmd = [a for a in cmd if a != "-c"]
     cmd[cmd.index("-o") + 1] = str(asm)
     subprocess.run(cmd + ["-S", "--cuda-device-only"], check=True, capture_output=True)
-    scratch = dict(re.findall(r"\.set (\S*gemm_w4a4_kernel\S*)\.private_seg_size, (\d+)", asm.read_text()))
-    tiles = {n: int(v) for n, v in scratch.items() if re.search(r"ILi[4-7]ELi4ELi4ELi1ELb[01]ELi2ELi2ELb0ELb0ELb1E", n)}
-    assert len(tiles) == 8 and not any(tiles.values()), tiles
+    scratch = re.findall(r"\.set (\S*)\.private_seg_size, (\d+)", asm.read_text())
+    found = {n: int(v) for n, v in scratch if re.search(kernels, n)}
+    assert len(found) == count and not any(found.values()), found
 
 
 def test_direct_loads_declare_their_register():
