@@ -512,8 +512,10 @@ def int4_twin(w: torch.Tensor, k: int) -> torch.Tensor | None:
 # loader: the calls of e3m2_form_pays run on them.  An entry lives as long as its INT4 weight and
 # is ignored once that weight is modified in place, like a twin's.
 _E3M2_FORMS: dict[int, tuple] = {}
-# A row count in place of e3m2_form_pays (None: the rule decides).
+# A row count in place of e3m2_form_pays (None: the rule decides), and the rows up to which no
+# call asks at all: seven per CU of the smallest device, one XCD of 32 CUs.
 E3M2_MIN_ROWS_K16384: int | None = None
+_FORM_ROWS_FLOOR = 7 * 32
 _CU_COUNT: dict[int, int] = {}
 
 
@@ -890,7 +892,7 @@ def _run(x: torch.Tensor, ws: list[torch.Tensor], tiled: bool, kind: str, gelu: 
     m = x.numel() // k
     if not gelu and k == 2048 and 1 <= m <= SMALL_M_MAX_ROWS and x.is_cuda:
         return _run_small(x, ws, k, m, tiled, kind, norm, residual)
-    if k == 16384 and len(ws) == 1 and norm is None and not tiled:
+    if k == 16384 and m > _FORM_ROWS_FLOOR and len(ws) == 1 and norm is None and not tiled:
         form = _form_for_rows(ws[0], k, m, x.device)
         if form is not None:
             if warm:  # a list that names the weight means what the call reads

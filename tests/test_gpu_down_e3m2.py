@@ -129,10 +129,10 @@ def test_weight_loaded_under_inference_mode(ext, cuda, monkeypatch):
     """No E3M2 form is kept for it, and its calls run on the INT4 weight."""
     from pi05_fast.w4a4.apply import load_time_weight
 
-    monkeypatch.setattr(ext, "E3M2_MIN_ROWS_K16384", 64)
+    monkeypatch.setattr(ext, "E3M2_MIN_ROWS_K16384", 256)
     gen = inp.generator(8400)
     packed = inp.random_packed(gen, 64, K)
-    x = inp.geglu_activations(gen, 100, K).to(cuda)
+    x = inp.geglu_activations(gen, 300, K).to(cuda)
     want = ext.int4_gemm(x, packed.to(cuda))
     with torch.inference_mode():
         w, shuffled = load_time_weight(packed, "layers.0.mlp.down_proj", K, 64, torch.device(cuda))
