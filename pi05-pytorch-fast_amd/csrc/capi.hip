@@ -646,7 +646,9 @@ namespace {
 // Tile counts and modes of the E3M2 main tile (16 mi x 256 outputs; GELU: 128 gate + up) for
 // M rows in ceil(M / 112) equal tiles: the smallest mi >= 4 that covers them (at 200 rows 7,
 // at 130 rows 5).  m-groups of the tile order: equal, at most 16 m-tiles (2.8 MB of codes at
-// K = 2048, which stay in an XCD's 4 MB L2).
+// K = 2048, which stay in an XCD's 4 MB L2).  At K = 16384 such a group's codes are 22 MB: there the
+// XCD's tiles share what they fetch only while they run over the same k blocks (at 6208 rows x 2048
+// columns 585 MB are read, 280 if every XCD fetched its tiles' operands once).
 void e3m2_main_tiles(w4a4::GemmParams& p, int64_t ntiles) {
   const int64_t m7 = cdiv(p.m, 112);
   p.ntiles = static_cast<int32_t>(ntiles);

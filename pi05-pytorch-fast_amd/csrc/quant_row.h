@@ -249,7 +249,7 @@ __device__ __forceinline__ void lane_stage(float (&v)[R], int lane) {
 //                 vector work and LDS phases better, but one row takes longer.
 // What bounds it is the chain of one row's phases (load, three register passes of 2 x 64
 // vector instructions per thread and stage pair, two transposes, one wide reduction) and how
-// many rows per CU hide each other's: at 6208 rows 305 MB move in 70 us (4.4 TB/s of the 5.2 a
+// many rows per CU hide each other's: at 6208 rows 305 MB move in 70 us (4.4 TB/s of the 4.9 a
 // copy reaches; 83 us before with three workgroup-wide transposes and rows written in
 // order); at 776 rows, three rows per CU, 14.8 us (17.0).  With four half rows per CU the
 // compiler has 128 registers and spills: 75.7 us at 6208 rows.
