@@ -598,7 +598,8 @@ def clear_weight_caches() -> None:
     and the E3M2 forms of K = 16384 weights), so that the next call rebuilds them from the
     current weights (twins and forms are not rebuilt: calls run on the weight given).
     Needed after writing a weight in place through ``.data`` (which bypasses the version
-    counter the caches check)."""
+    counter the caches check).  A graph captured before reads the dropped copies: capture it
+    again, as after any change of a weight that calls run on a copy of."""
     _MFMA_CACHE.clear()
     _INT4_TWINS.clear()
     _E3M2_FORMS.clear()

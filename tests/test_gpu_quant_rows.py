@@ -88,3 +88,21 @@ def test_unrotated_rows_match_oracle(ext, cuda, m, k):
     codes = orc.unpack_nibbles(inp.to_np(codes_from_fragment_major(q.cpu(), m, k)), k)
     want = -128 * codes[:, 1::2].astype(np.int64).sum(axis=1)
     assert np.array_equal(inp.to_np(qcorr_from_fragment_major(q.cpu(), m, k)), want)
+
+
+@pytest.mark.parametrize("k", [2112, 4096, 8192])
+def test_unrotated_infinities_and_nan(ext, cuda, k):
+    """Rows with infinities and NaN: a wave per row (600 rows) gives the codes, scales and row sums
+    of a workgroup per row (the first 500 of them alone)."""
+    from pi05_fast.w4a4.pack import codes_from_fragment_major, qcorr_from_fragment_major
+
+    x = _edge_rows(inp.generator(7700 + k), 600, k)
+    x[5, 9], x[12, 100], x[19, k - 1] = float("inf"), float("nan"), -float("inf")
+    x[26], x[33, ::2], x[40, ::3] = float("nan"), float("inf"), float("nan")
+    out = []
+    for m in (600, 500):
+        q, sa = ext.quantize(x[:m].to(cuda))
+        codes = inp.to_np(codes_from_fragment_major(q.cpu(), m, k))[:500]
+        out.append((codes, inp.to_np(sa).view(np.int32)[:500], inp.to_np(qcorr_from_fragment_major(q.cpu(), m, k))[:500]))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
