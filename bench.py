@@ -21,7 +21,7 @@ peak (GEMMs) or of HBM bandwidth (quantizers).  The graph removes host launch ga
 between the back-to-back kernels.  The non-W4A4 kernels of the forward (prefix attention,
 its K/V prep, RMSNorm) are timed the same way under `other_kernels`.
 The dominant kernel of the forward (the gate/up GEMM with its fused GELU-tanh*up
-epilogue, ~32% of the forward) is the `roofline` object; its `traffic` (HBM bytes per
+epilogue, ~29% of the forward) is the `roofline` object; its `traffic` (HBM bytes per
 launch) comes from the rocprofv3 FETCH_SIZE/WRITE_SIZE summary committed under profiles/.
 
 `in_forward` times the same kernels inside the real graph-replayed forward from their own
